@@ -105,51 +105,9 @@ LFDM_HD void step11(const PSet& P, const Derived& u, const K11& k, S11& s, doubl
                                    My[i]);
     }
     // computePowertrainRHS (dof11.cpp:607-749)
-    double torque_t;
-    double dcrank = 0.0;
-    const double gr = pick(P.gears, P.ngears, s.gear);
-    double shift_w;
-    if (P.tcbool) {
-        const double omega_out = xdiv<STRICT>(0.5 * (s.omega[0] + s.omega[1]), gr);
-        const double omega_in = s.crank;
-        double sr = 0;
-        bool rev = false;
-        if (!(omega_out < 1e-9 || omega_in < 1e-9)) {
-            sr = xdiv<STRICT>(omega_out, omega_in);
-            if (sr > 1.) {
-                sr = 1. - (sr - 1.);
-                rev = true;
-            }
-            if (sr < 0) sr = 0;
-        }
-        const double cf = map_y<STRICT>(P.cfmap, sr);
-        const double tr = map_y<STRICT>(P.trmap, sr);
-        const double q = xdiv<STRICT>(omega_in, cf);
-        double torque_in = -(q * q);
-        if (rev) torque_in = -torque_in;
-        const double torque_out = rev ? -torque_in : -tr * torque_in;
-        torque_t = xdiv<STRICT>(torque_out, gr);
-        if (s.u < 1e-9 && torque_t < 0) torque_t = 0;
-        dcrank = u.inv_ci * (drive_torque<STRICT>(P, k.tqs, throttle, s.crank) + torque_in);
-        shift_w = omega_out;
-    } else {
-        s.crank = xdiv<STRICT>(0.5 * (s.omega[0] + s.omega[1]), gr);
-        torque_t = xdiv<STRICT>(drive_torque<STRICT>(P, k.tqs, throttle, s.crank), gr);
-        if (s.u < 1e-9 && torque_t < 0) torque_t = 0;
-        shift_w = s.crank;
-    }
-    {
-        double up = P.shift[0].y, dn = P.shift[0].x;
-        for (int g = 1; g < P.ngears; ++g) {
-            up = (s.gear == g) ? P.shift[g].y : up;
-            dn = (s.gear == g) ? P.shift[g].x : dn;
-        }
-        if (shift_w > up) {
-            if (s.gear < P.ngears - 1) s.gear++;
-        } else if (shift_w < dn) {
-            if (s.gear > 0) s.gear--;
-        }
-    }
+    double torque_t, dcrank;
+    powertrain_torque<STRICT>(P, u, k.tqs, throttle, s.u, 0.5 * (s.omega[0] + s.omega[1]), s.crank, s.gear, torque_t,
+                              dcrank);
     // differentialSplit between the axles (dof11.cpp:271-311): 4WD splits with the bias rule
     // (rear axle in the "left" slot), else whichWheels picks the driven axle
     double eng[2];

@@ -119,6 +119,30 @@ struct TireOut18 {
     double fx[4], fy[4], My[4], rStat[4], xedot[4], yedot[4];
 };
 
+// computeVehRHS (dof18.cpp:1019-1078): chassis accelerations from the tire forces in the vehicle's axes.
+template <bool STRICT>
+LFDM_HD void chassis18(const PSet& P, const Derived& d, const K18& k, double u, double v, double wz, double wx,
+                       double phi, const double* fx, const double* fy, double& udot, double& vdot, double& wxdot,
+                       double& wzdot) {
+    const double E1 = k.neg_mt * wz * u + (fy[0] + fy[1] + fy[2] + fy[3]);
+    const double E2 = (fy[0] + fy[1]) * P.a - (fy[2] + fy[3]) * P.b + (fx[1] - fx[0]) * P.cf / 2 +
+                      (fx[3] - fx[2]) * P.cr / 2 + d.E2c * wz * u;
+    const double E3 = k.E3c * phi - d.kro * phi - d.bro * wx + k.hm * wz * u;
+    udot = wz * v + k.inv_mt * ((fx[0] + fx[1] + fx[2] + fx[3]) + d.Uc * (wz * wz) -
+                                                 k.two_hrc_m * wz * wx);
+    const double A1 = d.A1, A2 = k.A2, A3 = k.A3, jz = k.jz, jxz = P.jxz, mt = -k.neg_mt;
+    const double A3E1 = A3 * E1;
+    const double nv = E1 * d.jxz2 - k.A1A2 * E2 + A1 * E3 * jxz + A3 * E2 * jxz - A2 * E1 * jz - A3 * E3 * jz;
+    const double nwx = d.A1sq * E3 - k.A1A3 * E2 + A1 * E1 * jxz - A3E1 * jz + E2 * jxz * mt - E3 * jz * mt;
+    const double nwz = k.A3sq * E2 - k.A1A2 * E1 - k.A1A3 * E3 + A3E1 * jxz - A2 * E2 * mt + E3 * jxz * mt;
+    // the strict step divides by the determinant, formed as k18_init forms it (A1sq, A3sq and jxz2 are
+    // the products it squares)
+    const double denom = STRICT ? A2 * d.A1sq - 2. * A1 * A3 * jxz + jz * k.A3sq + mt * d.jxz2 - A2 * jz * mt : 0.0;
+    vdot = STRICT ? qdiv(nv, denom) : nv * k.rdenom;
+    wxdot = STRICT ? qdiv(nwx, denom) : nwx * k.rdenom;
+    wzdot = STRICT ? qdiv(nwz, denom) : nwz * k.rdenom;
+}
+
 // One half-implicit step (rhsFun order, dof18_halfImplicit.cpp:618-673; update :245-318).
 // STRICT: the reference's own quotients and transcendentals throughout (see dev_tire.h).  POS = false
 // leaves out the closing position update (position18).
@@ -188,26 +212,8 @@ LFDM_HD void step18(const PSet& P, const Derived& u, const K18& k, S18& s, doubl
         fx[i] = gx;
         fy[i] = gy;
     }
-    // computeVehRHS
-    const double wzu = s.wz * s.u;
-    const double E1 = k.neg_mt * s.wz * s.u + (fy[0] + fy[1] + fy[2] + fy[3]);
-    const double E2 = (fy[0] + fy[1]) * P.a - (fy[2] + fy[3]) * P.b + (fx[1] - fx[0]) * P.cf / 2 +
-                      (fx[3] - fx[2]) * P.cr / 2 + u.E2c * s.wz * s.u;
-    const double E3 = k.E3c * s.phi - u.kro * s.phi - u.bro * s.wx + k.hm * s.wz * s.u;
-    (void)wzu;
-    const double udot = s.wz * s.v + k.inv_mt * ((fx[0] + fx[1] + fx[2] + fx[3]) + u.Uc * (s.wz * s.wz) -
-                                                 k.two_hrc_m * s.wz * s.wx);
-    const double A1 = u.A1, A2 = k.A2, A3 = k.A3, jz = k.jz, jxz = P.jxz, mt = -k.neg_mt;
-    const double A3E1 = A3 * E1;
-    const double nv = E1 * u.jxz2 - k.A1A2 * E2 + A1 * E3 * jxz + A3 * E2 * jxz - A2 * E1 * jz - A3 * E3 * jz;
-    const double nwx = u.A1sq * E3 - k.A1A3 * E2 + A1 * E1 * jxz - A3E1 * jz + E2 * jxz * mt - E3 * jz * mt;
-    const double nwz = k.A3sq * E2 - k.A1A2 * E1 - k.A1A3 * E3 + A3E1 * jxz - A2 * E2 * mt + E3 * jxz * mt;
-    // the strict step divides by the determinant, formed as k18_init forms it (A1sq, A3sq and jxz2 are
-    // the products it squares)
-    const double denom = STRICT ? A2 * u.A1sq - 2. * A1 * A3 * jxz + jz * k.A3sq + mt * u.jxz2 - A2 * jz * mt : 0.0;
-    const double vdot = STRICT ? qdiv(nv, denom) : nv * k.rdenom;
-    const double wxdot = STRICT ? qdiv(nwx, denom) : nwx * k.rdenom;
-    const double wzdot = STRICT ? qdiv(nwz, denom) : nwz * k.rdenom;
+    double udot, vdot, wxdot, wzdot;
+    chassis18<STRICT>(P, u, k, s.u, s.v, s.wz, s.wx, s.phi, fx, fy, udot, vdot, wxdot, wzdot);
     // Half-implicit update (dof18_halfImplicit.cpp:262-305)
 #pragma unroll
     for (int i = 0; i < 4; ++i) {

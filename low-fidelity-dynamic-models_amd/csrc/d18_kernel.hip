@@ -5,6 +5,7 @@ namespace lfdm {
 
 hipError_t launch_d18(const Launch& L, int block, hipStream_t stream) {
     if (L.S <= 0 || L.nsteps <= 0) return hipSuccess;
+    if (L.lanes > 1 && !L.strict) return launch_d18_group(L, block, stream);
     return kern::launch_model<kern::M18>(L, block, stream);
 }
 

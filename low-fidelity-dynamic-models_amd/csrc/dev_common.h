@@ -93,18 +93,28 @@ LFDM_HD double qsqrt(double x) {
 // square of the hardware estimate's) makes the correctly rounded value for all but operands within a
 // minute fraction of an ulp of a rounding boundary.  Same operand ranges as qdiv and qsqrt.  Host
 // builds use `/` and sqrt.
-LFDM_HD double fdiv(double n, double d) {
+LFDM_HD double fdiv_rcp(double d) {  // fdiv's once-refined reciprocal of the divisor
 #if defined(__HIP_DEVICE_COMPILE__)
-    double r = __builtin_amdgcn_rcp(d);
+    const double r = __builtin_amdgcn_rcp(d);
     const double e = __builtin_fma(-d, r, 1.0);
-    r = __builtin_fma(r, e, r);
+    return __builtin_fma(r, e, r);
+#else
+    return 1.0 / d;
+#endif
+}
+
+LFDM_HD double fdiv_by(double n, double d, double r) {  // fdiv(n, d), r = fdiv_rcp(d)
+#if defined(__HIP_DEVICE_COMPILE__)
     const double q = n * r;
     const double rem = __builtin_fma(-d, q, n);
     return __builtin_fma(rem, r, q);
 #else
+    (void)r;
     return n / d;
 #endif
 }
+
+LFDM_HD double fdiv(double n, double d) { return fdiv_by(n, d, fdiv_rcp(d)); }
 
 LFDM_HD double frcp(double d) {
 #if defined(__HIP_DEVICE_COMPILE__)

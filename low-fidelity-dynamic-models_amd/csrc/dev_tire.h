@@ -134,13 +134,11 @@ template <bool STRICT = false>
 LFDM_HD void tmeasy_eval(const TireP& t, const Derived& u, double qy1, double qy2, double delta, double tan_delta,
                          double fz, double rStat, double vsx, double vsy, double xe, double ye, double omega,
                          TireEval& w) {
-    if (fz <= t.fzRdynco) {
-        w.rdynco = t.rdyncoPn + u.lrd * ((STRICT ? qdiv(fz, t.pn) : fz * u.inv_pn) - 1.);
-        w.drd = u.lrd * u.inv_pn;
-    } else {
-        w.rdynco = t.rdyncoCrit;
-        w.drd = 0.0;
-    }
+    // selected, not branched to: the branch's parameter loads would each wait for the scalar cache
+    const bool below = fz <= t.fzRdynco;
+    const double rd_below = t.rdyncoPn + u.lrd * ((STRICT ? qdiv(fz, t.pn) : fz * u.inv_pn) - 1.);
+    w.rdynco = below ? rd_below : t.rdyncoCrit;
+    w.drd = below ? u.lrd * u.inv_pn : 0.0;
     w.r_eff = w.rdynco * t.r0 + (1. - w.rdynco) * rStat;
     w.vsx2 = vsx - (omega * w.r_eff);
     w.aom = fabs(omega);
@@ -297,11 +295,8 @@ LFDM_HD void tmeasy_nr_core(const TireP& t, const Derived& u, double qy1, double
                                                double tan_delta, double fz, double rStat, double vsx, double vsy,
                                                double omega, double& fx, double& fy, double& My) {
     const double vsx_in = vsx;
-    double rdynco;
-    if (fz <= t.fzRdynco)
-        rdynco = t.rdyncoPn + u.lrd * ((STRICT ? qdiv(fz, t.pn) : fz * u.inv_pn) - 1.);
-    else
-        rdynco = t.rdyncoCrit;
+    const double rd_below = t.rdyncoPn + u.lrd * ((STRICT ? qdiv(fz, t.pn) : fz * u.inv_pn) - 1.);
+    const double rdynco = fz <= t.fzRdynco ? rd_below : t.rdyncoCrit;
     const double r_eff = rdynco * t.r0 + (1. - rdynco) * rStat;
     vsx = vsx - (omega * r_eff);
     const double vta = r_eff * fabs(omega) + 0.01;
@@ -406,24 +401,20 @@ LFDM_HD double drive_torque(const PSet& P, double tqs, double throttle, double w
     return tq * throttle + map_y<STRICT>(P.losses, w);
 }
 
-// computePowertrainRHS of the four-wheel models (dof18.cpp:675-845, dof24.cpp:1338-1509): torque
-// converter or slaved crank, gear shift for the next step, axle and differential split, wheel
-// accelerations.  Updates crank (without a converter) and gear; returns dOm, eng and dcrank.
+// The part of computePowertrainRHS (dof18.cpp:675-800, dof24.cpp:1338-1462, dof11.cpp:607-720) ahead of the axles: torque
+// converter or slaved crank and the gear shift for the next step, from the wheels' mean speed.
+// Updates crank (without a converter) and gear; returns the shaft torque and dcrank.
 template <bool STRICT>
-LFDM_HD void powertrain4(const PSet& P, const Derived& u, double tqs, double maxBrake,
-                                            double throttle, double braking, double vel_u, double& crank, int& gear,
-                                            const double* omega, const double* fx, const double* rStat,
-                                            const double* My, double* dOm, double* eng, double& dcrank) {
-    double torque_t;
+LFDM_HD void powertrain_torque(const PSet& P, const Derived& u, double tqs, double throttle, double vel_u, double mean,
+                               double& crank, int& gear, double& torque_t, double& dcrank) {
     dcrank = 0.0;
-    const double osum = omega[0] + omega[1] + omega[2] + omega[3];
     const double gr = pick(P.gears, P.ngears, gear);
     double shift_w;
     // the quotients by the gear ratio stay divisions in the fast form too: the converter's speed ratio
     // omega_out / crank is exactly 1 at a crank speed set from the same quotient, and the model's
     // reverse-flow branch (sr > 1) flips with one ulp there
     if (P.tcbool) {
-        const double omega_out = xdiv<STRICT>(0.25 * osum, gr);
+        const double omega_out = xdiv<STRICT>(mean, gr);
         const double omega_in = crank;
         double sr = 0;
         bool rev = false;
@@ -446,7 +437,7 @@ LFDM_HD void powertrain4(const PSet& P, const Derived& u, double tqs, double max
         dcrank = u.inv_ci * (drive_torque<STRICT>(P, tqs, throttle, crank) + torque_in);
         shift_w = omega_out;
     } else {
-        crank = xdiv<STRICT>(0.25 * osum, gr);
+        crank = xdiv<STRICT>(mean, gr);
         torque_t = xdiv<STRICT>(drive_torque<STRICT>(P, tqs, throttle, crank), gr);
         if (vel_u < 1e-9 && torque_t < 0) torque_t = 0;
         shift_w = crank;
@@ -463,7 +454,10 @@ LFDM_HD void powertrain4(const PSet& P, const Derived& u, double tqs, double max
             if (gear > 0) gear--;
         }
     }
-    double tf, trr;
+}
+
+// The shaft torque's share of the front and the rear axle.
+LFDM_HD void axle_torques(const PSet& P, double torque_t, double& tf, double& trr) {
     if (P.driveType) {
         tf = torque_t * 0.5;
         trr = torque_t * 0.5;
@@ -474,6 +468,20 @@ LFDM_HD void powertrain4(const PSet& P, const Derived& u, double tqs, double max
         tf = torque_t;
         trr = 0;
     }
+}
+
+// computePowertrainRHS of the four-wheel models (dof18.cpp:675-845, dof24.cpp:1338-1509): torque
+// converter or slaved crank, gear shift for the next step, axle and differential split, wheel
+// accelerations.  Updates crank (without a converter) and gear; returns dOm, eng and dcrank.
+template <bool STRICT>
+LFDM_HD void powertrain4(const PSet& P, const Derived& u, double tqs, double maxBrake,
+                                            double throttle, double braking, double vel_u, double& crank, int& gear,
+                                            const double* omega, const double* fx, const double* rStat,
+                                            const double* My, double* dOm, double* eng, double& dcrank) {
+    double torque_t, tf, trr;
+    const double osum = omega[0] + omega[1] + omega[2] + omega[3];
+    powertrain_torque<STRICT>(P, u, tqs, throttle, vel_u, 0.25 * osum, crank, gear, torque_t, dcrank);
+    axle_torques(P, torque_t, tf, trr);
     diff_split<STRICT>(tf, omega[0], omega[1], eng[0], eng[1]);
     diff_split<STRICT>(trr, omega[2], omega[3], eng[2], eng[3]);
     const double bt = maxBrake * braking;

@@ -12,6 +12,7 @@
 #include "d11_device.h"
 #include "d18_device.h"
 #include "d24_device.h"
+#include "group.h"
 #include "kernels.h"
 
 namespace lfdm {
@@ -97,6 +98,7 @@ struct M18 {
     static constexpr int kCh = 13;
     static constexpr int kWaves = kMaxWaves18;
     static constexpr bool kKInLds = true;
+    static constexpr int kLanes = 1;  // lanes per vehicle
     template <bool NR>
     struct R {
         static constexpr int kTire = NR ? 11 : 15, kVeh = 4 * kTire, om = NR ? 0 : 4;
@@ -172,6 +174,7 @@ struct M11 {
     static constexpr int kCh = 9;
     static constexpr int kWaves = kMaxWaves11;
     static constexpr bool kKInLds = true;
+    static constexpr int kLanes = 1;  // lanes per vehicle
     template <bool NR>
     struct R {
         static constexpr int kTire = NR ? 11 : 15, kVeh = 2 * kTire, om = NR ? 0 : 4;
@@ -247,6 +250,7 @@ struct M24 {
     static constexpr int kCh = 15;
     static constexpr int kWaves = kMaxWaves24;
     static constexpr bool kKInLds = true;
+    static constexpr int kLanes = 1;  // lanes per vehicle
     template <bool NR>
     struct R {
         static constexpr int kTire = NR ? 19 : 23, kSus = 4 * kTire, kVeh = kSus + 4 * 24, om = NR ? 0 : 4;
@@ -345,6 +349,17 @@ struct M24 {
     }
 };
 
+// The powertrain's maps of P into tab[kGroupMapEntries], by one wavefront.
+__device__ __forceinline__ void stage_maps(const PSet& P, MapXY* tab, int lane) {
+#pragma unroll
+    for (int id = 0; id < kGroupMaps; ++id)
+        if (lane < kMaxMap) tab[id * kMaxMap + lane] = group_map(P, id).e[lane];
+    // the lanes that read an entry belong to the wavefront that wrote it
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
 // Occupancy of the integration kernels (waves per SIMD).  Each model has a default, M::kWaves, the
 // most waves per SIMD it is built for: on large fleets more resident waves hide more FP64 latency
 // than the register spills of a smaller budget cost, up to four for the 11-DOF step (five run 2 %
@@ -358,7 +373,9 @@ struct M24 {
 // occupancy only).
 template <class M, bool NR, int MODE, int W, bool STRICT, class F = NoControls>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(W, W))) void integrate(Launch L, F f) {
-    const int slot = blockIdx.x * blockDim.x + threadIdx.x;
+    // M::kLanes neighbouring lanes run one vehicle (group.h); a wavefront's vehicles are all of one
+    // 64-slot block, so its parameter set stays uniform
+    const int slot = (int)((blockIdx.x * blockDim.x + threadIdx.x) / M::kLanes);
     const int wave = uniform(slot >> 6);
     if (wave * kWave >= L.S) return;
     // steps of this lane and of its wavefront in this launch: all of them, or up to the vehicle's
@@ -381,9 +398,16 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(W, W))) voi
     typename M::K k_reg;
     typename M::K& k = M::kKInLds ? reinterpret_cast<typename M::K*>(lfdm_k_lds)[threadIdx.x] : k_reg;
     typename M::S s;
+    if constexpr (M::kLanes > 1) s.q = (int)(threadIdx.x % M::kLanes);
     M::template load<NR>(L.state, S, slot, s, k);
     const Derived& u = P.d;
-    M::kinit(P, L.ovr + slot, S, k);
+    if constexpr (M::kLanes > 1) {
+        MapXY* tab = reinterpret_cast<MapXY*>(lfdm_k_lds) + (threadIdx.x / kWave) * kGroupMapEntries;
+        stage_maps(P, tab, (int)(threadIdx.x % kWave));
+        M::kinit(P, L.ovr + slot, S, tab, s, k);
+    } else {
+        M::kinit(P, L.ovr + slot, S, k);
+    }
     const int user = L.slot_user[slot];
     const int uv = user >= 0 ? user : 0;  // padding lanes read vehicle 0's controls
     CtrlState<MODE> cs;
@@ -403,9 +427,15 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(W, W))) voi
     for (int kk = 0; kk < wsteps - 1; ++kk) {
         if constexpr (M::kKInLds) LFDM_RELOAD_MEMORY();
         if (kk < my - 1) {
-            if (kk != clean) M::template position<STRICT>(s, dt);  // the same branch on every lane
-            const Ctl c = controls_at<MODE>(L, P, cs, uv, kk, t, f);
-            M::template step<NR, false, STRICT, false>(P, u, k, s, c, dt, nullptr);
+            // kk != clean: the same branch on every lane
+            if constexpr (M::kLanes > 1) {
+                const Ctl c = controls_at<MODE>(L, P, cs, uv, kk, t, f);
+                M::template step<NR, false>(P, u, k, s, c, dt, kk != clean, nullptr);
+            } else {
+                if (kk != clean) M::template position<STRICT>(s, dt);
+                const Ctl c = controls_at<MODE>(L, P, cs, uv, kk, t, f);
+                M::template step<NR, false, STRICT, false>(P, u, k, s, c, dt, nullptr);
+            }
             pend = true;
             t = t + dt;
         }
@@ -426,7 +456,8 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(W, W))) voi
         typename M::X x;
         CtrlState<MODE> cl;
         const Ctl c = controls_at<MODE>(L, P, my == wsteps ? cs : cl, uv, my - 1, t, f);
-        M::template step<NR, true, STRICT, false>(P, u, k, s, c, dt, &x);
+        if constexpr (M::kLanes > 1) M::template step<NR, true>(P, u, k, s, c, dt, false, &x);
+        else M::template step<NR, true, STRICT, false>(P, u, k, s, c, dt, &x);
         M::template position<STRICT>(s, dt);
         t = t + dt;
         M::template store<NR>(L.state, S, slot, P, s, k, x);
@@ -445,15 +476,16 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(W, W))) voi
 }
 
 // Dynamic LDS of an integration launch of `block` threads: one K per lane where the model keeps its
-// per-vehicle constants in LDS.
+// per-vehicle constants in LDS; the lane-group kernels' maps, one copy per wavefront.
 template <class M>
 constexpr size_t k_lds_bytes(int block) {
+    if (M::kLanes > 1) return (size_t)(block / kWave) * kGroupMapEntries * sizeof(MapXY);
     return M::kKInLds ? (size_t)block * sizeof(typename M::K) : 0;
 }
 
 template <class M, bool NR, int W, bool STRICT>
 hipError_t launch_mode(const Launch& L, int block, hipStream_t stream) {
-    const int grid = (L.S + block - 1) / block;
+    const int grid = (int)(((long long)L.S * M::kLanes + block - 1) / block);
     const size_t lds = k_lds_bytes<M>(block);
     switch (L.mode) {
         case kCtrlTable: hipLaunchKernelGGL((integrate<M, NR, kCtrlTable, W, STRICT>), grid, block, lds, stream, L, NoControls{}); break;

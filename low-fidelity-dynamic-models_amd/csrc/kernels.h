@@ -23,6 +23,35 @@ __device__ __forceinline__ const PSet& pset_at(const PSet* sets, int i) {
 // occupancy; the maximum is the default on fleets of more than one wavefront per SIMD).
 constexpr int kMaxWaves11 = 4, kMaxWaves18 = 3, kMaxWaves24 = 2;
 
+// Lanes per vehicle and waves per SIMD of the kernel a fleet of S slots runs on a device of `simds` SIMDs
+// (waves 0: the model's most).  A lone wavefront on a SIMD leaves most of its cycles unused, and a
+// fleet of few wavefronts leaves SIMDs idle, so such fleets spread each vehicle over a group of lanes
+// (csrc/group.h): every lane then has one or two tires instead of four and shares the map lookups and
+// angles.  Measured per step (TMeasy fleets, microseconds; one lane / two / four):
+//   18-DOF  16,384 vehicles  7.8 / 4.0 / 2.8    32,768  8.1 / 4.2 / 4.3    65,536  8.3 / 6.3 / 7.7
+//   24-DOF  16,384 vehicles  9.9 / 5.4 / 3.6    32,768 10.3 / 5.3 / 5.1    65,536 10.3 / 8.7 / 9.8
+//   11-DOF  16,384 vehicles  4.9 / 2.6          32,768  5.5 / 2.8          65,536  5.7 / 4.0
+// So: four lanes while they make at most two wavefronts per SIMD, two lanes while they do, and one lane
+// beyond (at 131,072 18-DOF vehicles two lanes would take two rounds of 6.3 against 10.8).  The kernels are
+// built for the wavefronts per SIMD they make, which keeps the dispatcher from stacking two on one SIMD
+// while another is idle.  One-lane fleets of w wavefronts per SIMD, w below the model's most, run the
+// kernel built for w for the same reason.
+struct KernelChoice {
+    int lanes, waves;
+};
+
+inline KernelChoice choose_kernel(int dof, long long S, int simds, bool strict) {
+    const long long wf = S / kWave;
+    if (simds <= 0 || wf <= 0) return {1, 0};
+    const auto per = [&](int lanes) { return (wf * lanes + simds - 1) / simds; };
+    if (!strict) {
+        if (dof != 11 && per(4) <= 2) return {4, (int)per(4)};
+        if (per(2) <= 2) return {2, dof == 11 ? (int)per(2) : 2};
+    }
+    const int most = dof == 11 ? kMaxWaves11 : dof == 18 ? kMaxWaves18 : kMaxWaves24;
+    return {1, per(1) < most ? (int)per(1) : 0};
+}
+
 struct Launch {
     const PSet* sets;       // parameter sets
     const int* wave_set;   // set index of every 64-slot wavefront
@@ -47,6 +76,7 @@ struct Launch {
     const int* wave_hmax;
     int step_base;
     int waves;  // waves per SIMD of the kernel: 1 up to the model's maximum, or 0 for its default
+    int lanes;  // lanes per vehicle: 0 or 1 the one-lane kernels, 2 or 4 the lane-group kernels (not for strict)
     int strict;  // 1: the step with the reference's own quotients and transcendentals (LFDM_ARITH_STRICT)
 };
 
@@ -55,6 +85,9 @@ struct Launch {
 hipError_t launch_d11(const Launch& L, int block, hipStream_t stream);
 hipError_t launch_d18(const Launch& L, int block, hipStream_t stream);
 hipError_t launch_d24(const Launch& L, int block, hipStream_t stream);
+hipError_t launch_d11_group(const Launch& L, int block, hipStream_t stream);
+hipError_t launch_d24_group(const Launch& L, int block, hipStream_t stream);
+hipError_t launch_d18_group(const Launch& L, int block, hipStream_t stream);
 
 // Differentiation form (18-DOF TMeasy).  Forward: from the record state, nsteps steps with per-step
 // controls ctrl[nsteps][3][n_user]; writes xy[nsteps][2][n_user] (position after each step) and

@@ -21,7 +21,7 @@ struct MapXY {
 
 struct Map {
     int n;
-    int pad;
+    int sorted;  // abscissae ascend (an interval can be walked to from its neighbours)
     MapXY e[kMaxMap];
 };
 

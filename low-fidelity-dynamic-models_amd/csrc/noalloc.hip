@@ -173,11 +173,9 @@ extern "C" int lfdm_integrate_noalloc(int dof, const double* flat, int len, int 
         L.n_user = (int)n;
         L.mode = kCtrlSteps;
         L.nr = tire_type == LFDM_TIRE_TMEASYNR;
-        {  // the handle path's rule: the wavefronts per SIMD the fleet fills, below the model's default
-            const long long per = simds > 0 ? ((long long)(S / kWave) + simds - 1) / simds : 0;
-            const int wmax = dof == 11 ? kMaxWaves11 : dof == 18 ? kMaxWaves18 : kMaxWaves24;
-            L.waves = (per > 0 && per < wmax) ? (int)per : 0;
-        }
+        const KernelChoice c = choose_kernel(dof, S, simds, arith == LFDM_ARITH_STRICT);
+        L.lanes = c.lanes;
+        L.waves = c.waves;
         L.strict = arith == LFDM_ARITH_STRICT;
         const hipError_t e = dof == 11 ? launch_d11(L, kWave, st) : dof == 18 ? launch_d18(L, kWave, st)
                                                                             : launch_d24(L, kWave, st);

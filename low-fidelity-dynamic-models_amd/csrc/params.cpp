@@ -347,12 +347,14 @@ struct Rd {
         if (n > kMaxMap) { err = std::string("map ") + name + " has more than " + std::to_string(kMaxMap) + " entries"; ok = false; return false; }
         if (required && n == 0) { err = std::string("map ") + name + " is empty"; ok = false; return false; }
         m.n = n;
-        m.pad = 0;
         for (int k = 0; k < n; ++k) {
             m.e[k].x = next();
             m.e[k].y = next();
         }
         for (int k = n; k < kMaxMap; ++k) m.e[k].x = m.e[k].y = 0.0;
+        m.sorted = 1;
+        for (int k = 0; k + 1 < n; ++k)
+            if (!(m.e[k].x <= m.e[k + 1].x)) m.sorted = 0;
         return ok;
     }
 };

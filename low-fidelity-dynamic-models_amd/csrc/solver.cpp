@@ -482,13 +482,10 @@ Launch make_launch(lfdm_solver* h, int mode, double t0, int nsteps, double cs = 
         L.wave_hmax = h->d_wave_hmax;
         L.step_base = (int)std::llround(t0 / h->step);
     }
-    // a fleet of at most w wavefronts per SIMD, w below the model's default, runs the kernels built for
-    // w waves per SIMD: their larger register budget spills less, and no SIMD can take more of the
-    // fleet's wavefronts than w (at two per SIMD, the 18-DOF kernel built for three ran 1.3x slower)
-    const int simds = simd_count(h);
-    const long long per = simds > 0 ? ((long long)h->S / kWave + simds - 1) / simds : 0;
-    L.waves = (per > 0 && per < max_waves(h->dof)) ? (int)per : 0;
     L.strict = h->arith == LFDM_ARITH_STRICT ? 1 : 0;
+    const KernelChoice c = choose_kernel(h->dof, h->S, simd_count(h), L.strict != 0);
+    L.lanes = c.lanes;
+    L.waves = c.waves;
     return L;
 }
 
@@ -597,7 +594,11 @@ std::vector<Launch> run_launches(lfdm_solver* h, int nsteps, int spl, int waves,
         const int n = std::min(spl > 0 ? spl : nsteps, nsteps - done);
         Launch L = make_launch(h, h->ctrl_mode, t, n, 0, 0, 0, steps ? steps + (size_t)done * row : nullptr);
         if (L.horizon) L.step_base = done;
-        if (waves > 0) L.waves = waves;
+        // 1 on a fleet of at most one wavefront per SIMD is the automatic choice (lane groups)
+        if (waves > 1 || (waves == 1 && L.lanes == 1)) {
+            L.lanes = 1;
+            L.waves = waves;
+        }
         r.push_back(L);
         for (int k = 0; k < n; ++k) t += h->step;
         done += n;

@@ -1,0 +1,155 @@
+// Host build of the lane-group steps (csrc/d{11,18,24}_group.h) against the one-lane steps they must equal
+// bit for bit.  A group's lanes run as threads that meet at every exchange (group.h's host_group_exchange),
+// so the same code runs here as on the device, lane by lane.  Built by the Makefile's `groupstep`; loaded
+// by tests/test_group_host.py.
+#include <atomic>
+#include <cstdio>
+#include <string>
+#include <thread>
+#include <vector>
+
+#include "../../low-fidelity-dynamic-models_amd/csrc/integrate_group.h"
+#include "../../low-fidelity-dynamic-models_amd/csrc/params.h"
+
+using namespace lfdm;
+
+namespace {
+
+// The lanes of one group: every lane posts its value, waits for all, reads the one it wants, waits again.
+struct Meeting {
+    explicit Meeting(int n) : n(n) {}
+    void meet() {
+        const int turn = round.load(std::memory_order_acquire);
+        if (arrived.fetch_add(1, std::memory_order_acq_rel) + 1 == n) {
+            arrived.store(0, std::memory_order_relaxed);
+            round.fetch_add(1, std::memory_order_acq_rel);
+        } else {
+            while (round.load(std::memory_order_acquire) == turn) std::this_thread::yield();
+        }
+    }
+    double exchange(int lane, double v, int q) {
+        post[lane] = v;
+        meet();
+        const double r = post[q];
+        meet();
+        return r;
+    }
+    const int n;
+    double post[4];
+    std::atomic<int> arrived{0}, round{0};
+};
+
+thread_local Meeting* t_meeting;
+thread_local int t_lane;
+
+double exchange(double v, int g, int q) {
+    return t_meeting->exchange(t_lane, v, (t_lane & ~(g - 1)) + q);  // g 2 among four lanes: this lane's pair
+}
+
+struct Run {
+    const PSet& P;
+    const double* ovr;  // [7][n]
+    const double* ctrl;  // [nsteps][3][n]
+    int n, rec, nsteps;
+    double dt;
+};
+
+kern::Ctl ctl(const Run& r, int i, int j) {
+    const double* c = r.ctrl + (size_t)j * 3 * r.n + i;
+    return {c[0], c[r.n], c[2 * r.n]};
+}
+
+// Both mirror the integration kernel's loop: every step but the last keeps the carried state and leaves its
+// position update to the next, the last also returns the full record.
+template <class M, bool NR>
+void one_lane(const Run& r, double* st, int i) {
+    typename M::S s;
+    typename M::K k;
+    typename M::X x;
+    M::template load<NR>(st, r.n, i, s, k);
+    M::kinit(r.P, r.ovr + i, r.n, k);
+    for (int j = 0; j < r.nsteps; ++j) {
+        if (j > 0) M::template position<false>(s, r.dt);
+        if (j + 1 < r.nsteps)
+            M::template step<NR, false, false, false>(r.P, r.P.d, k, s, ctl(r, i, j), r.dt, nullptr);
+        else
+            M::template step<NR, true, false, false>(r.P, r.P.d, k, s, ctl(r, i, j), r.dt, &x);
+    }
+    M::template position<false>(s, r.dt);
+    M::template store<NR>(st, r.n, i, r.P, s, k, x);
+}
+
+template <class M, bool NR>
+void group(const Run& r, double* st, int i) {
+    std::vector<MapXY> tab(kGroupMapEntries);
+    for (int id = 0; id < kGroupMaps; ++id)
+        for (int e = 0; e < kMaxMap; ++e) tab[id * kMaxMap + e] = group_map(r.P, id).e[e];
+    Meeting all(M::kLanes);
+    std::vector<std::thread> lanes;
+    for (int q = 0; q < M::kLanes; ++q)
+        lanes.emplace_back([&, q] {
+            t_meeting = &all;
+            t_lane = q;
+            host_group_exchange = exchange;
+            typename M::S s;
+            typename M::K k;
+            typename M::X x;
+            s.q = q;
+            M::template load<NR>(st, r.n, i, s, k);
+            M::kinit(r.P, r.ovr + i, r.n, tab.data(), s, k);
+            for (int j = 0; j + 1 < r.nsteps; ++j)
+                M::template step<NR, false>(r.P, r.P.d, k, s, ctl(r, i, j), r.dt, j > 0, nullptr);
+            if (r.nsteps > 1) M::template position<false>(s, r.dt);
+            M::template step<NR, true>(r.P, r.P.d, k, s, ctl(r, i, r.nsteps - 1), r.dt, false, &x);
+            M::template position<false>(s, r.dt);
+            all.meet();  // every lane has read the record before any writes it
+            M::template store<NR>(st, r.n, i, r.P, s, k, x);
+        });
+    for (std::thread& t : lanes) t.join();
+}
+
+template <class M, bool NR, bool GROUP>
+void run(const Run& r, const double* init, double* fin) {
+    std::vector<double> st((size_t)r.rec * r.n);
+    for (int i = 0; i < r.n; ++i)
+        for (int f = 0; f < r.rec; ++f) st[(size_t)f * r.n + i] = init[(size_t)i * r.rec + f];
+    for (int i = 0; i < r.n; ++i) {
+        if constexpr (GROUP) group<M, NR>(r, st.data(), i);
+        else one_lane<M, NR>(r, st.data(), i);
+    }
+    for (int i = 0; i < r.n; ++i)
+        for (int f = 0; f < r.rec; ++f) fin[(size_t)i * r.rec + f] = st[(size_t)f * r.n + i];
+}
+
+template <class M, bool GROUP>
+void pick_tire(const Run& r, int nr, const double* init, double* fin) {
+    if (nr) run<M, true, GROUP>(r, init, fin);
+    else run<M, false, GROUP>(r, init, fin);
+}
+
+}  // namespace
+
+// n vehicles, nsteps >= 1 steps on `lanes` lanes per vehicle (1, 2 or 4): final records into fin[n][rec].
+// walks receives whether the group's map walk serves this parameter set.
+extern "C" int group_step_run(int dof, int nr, int lanes, const double* flat, int len, const double* ovr,
+                              const double* init, int n, int rec, int nsteps, const double* ctrl, double dt,
+                              double* fin, int* walks) {
+    PSet P;
+    std::string e;
+    if (!pset_from_flat(dof, flat, len, nr, P, e)) {
+        std::fprintf(stderr, "%s\n", e.c_str());
+        return -1;
+    }
+    *walks = group_walks(P) ? 1 : 0;
+    const Run r{P, ovr, ctrl, n, rec, nsteps, dt};
+    if (dof == 11 && lanes == 1) pick_tire<kern::M11, false>(r, nr, init, fin);
+    else if (dof == 11 && lanes == 2) pick_tire<kern::M11g, true>(r, nr, init, fin);
+    else if (dof == 18 && lanes == 1) pick_tire<kern::M18, false>(r, nr, init, fin);
+    else if (dof == 18 && lanes == 2) pick_tire<kern::M18g<2>, true>(r, nr, init, fin);
+    else if (dof == 18 && lanes == 4) pick_tire<kern::M18g<4>, true>(r, nr, init, fin);
+    else if (dof == 24 && lanes == 1) pick_tire<kern::M24, false>(r, nr, init, fin);
+    else if (dof == 24 && lanes == 2) pick_tire<kern::M24g<2>, true>(r, nr, init, fin);
+    else if (dof == 24 && lanes == 4) pick_tire<kern::M24g<4>, true>(r, nr, init, fin);
+    else return -2;
+    return 0;
+}

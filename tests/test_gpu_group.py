@@ -1,0 +1,52 @@
+"""Small fleets on the GPU run the lane-group kernels (two or four lanes per vehicle); results have the bits
+of the one-lane kernels, which a fleet bucket set to two waves per SIMD runs at any size."""
+import os
+
+import numpy as np
+import pytest
+
+from conftest import DATA
+
+import lfdm_amd
+from lfdm_amd import workloads as W
+from lfdm_amd.solver import Fleet, SolverHalfImplicitGPU, TMeasy, TMeasyNr
+
+pytestmark = pytest.mark.gpu
+
+# One vehicle, around a wavefront, and either side of the sizes where the choice changes on 1,024 SIMDs
+# (four lanes up to 16,384 at one and 32,768 at two wavefronts per SIMD, two lanes up to 65,536).
+SIZES = [1, 65, 16384, 16385, 32769, 65536, 65537]
+
+
+def fleet(dof, nr, n):
+    d = os.path.join(DATA, f"{dof}dof", "Sedan" if nr else "HMMWV")
+    flat = lfdm_amd.params_from_json(dof, f"{d}/vehicle.json", f"{d}/tmeasyNr.json" if nr else f"{d}/tmeasy.json",
+                                     f"{d}/suspension.json" if dof == 24 else None, int(nr))
+    fl = W.knot_fleet(n, flat, seed=n, dof=dof, tire_nr=nr)
+    s = SolverHalfImplicitGPU(dof, n)
+    s.construct_flat(flat, n, None, TMeasyNr if nr else TMeasy)
+    s.set_overrides(fl["ovr"])
+    s.initialize_batch(W.initial_speed_records(n, flat, dof, seed=3, tire_nr=nr))
+    s.set_controls_knots(fl["ns"], fl["ds"], fl["np"], fl["dp"], fl["knots"])
+    s.set_horizons(np.random.default_rng(n).integers(0, 61, n))
+    return s
+
+
+@pytest.mark.parametrize("n", SIZES)
+@pytest.mark.parametrize("dof,nr", [(11, False), (11, True), (18, False), (18, True), (24, False), (24, True)])
+def test_lane_groups_give_the_one_lane_bits(dof, nr, n):
+    s = fleet(dof, nr, n)
+    init = s.get_states()
+    with Fleet([s]) as f:
+        f.set_config(0, 64, 0, 2)  # one lane per vehicle
+        f.run(60)
+        f.synchronize()
+        ref = s.get_states()
+        s.set_states(init)
+        f.set_config(0, 128, 25, 0)  # the automatic choice, in three launches of two-wavefront blocks
+        f.run(60)
+        f.synchronize()
+        got = s.get_states()
+    s.close()
+    assert n < 64 or not np.array_equal(ref, init)
+    np.testing.assert_array_equal(got, ref)

@@ -1,0 +1,138 @@
+"""The lane-group steps compiled for the host (tests/cpp/group_step.cpp) against the one-lane step.
+
+A lane-group kernel must give a vehicle the same bits as the one-lane kernel: whatever the vehicle (four-,
+front- and rear-wheel drive, with and without a torque converter, linear and tabled steering, throttle-scaled
+torque map), the tire model, and the shape of its powertrain maps, including those the map walk leaves to
+the scan.  Every lane runs as a thread here, with the device code's exchanges.
+"""
+import ctypes
+import os
+
+import numpy as np
+import pytest
+
+from conftest import DATA, ROOT
+
+import lfdm_amd
+import lfdm_oracle as O
+from lfdm_amd import workloads as W
+
+LIB = os.path.join(ROOT, "low-fidelity-dynamic-models_amd", "lfdm_amd", "libgroup_step.so")
+N, STEPS = 6, 400
+
+
+def params(dof, veh, tire, nr):
+    d = os.path.join(DATA, f"{dof}dof")
+    sus = f"{d}/{veh.split('/')[0]}/suspension.json" if dof == 24 else None
+    return lfdm_amd.params_from_json(dof, f"{d}/{veh}", f"{d}/{tire}", sus, int(nr))
+
+
+def maps_at(flat, dof):
+    """Start of each map (its entry count) in the flat vector: shift, steer, torque, losses, cf, tr."""
+    i = W.FLAT[dof]["gears"]
+    i += 1 + int(flat[i])
+    out = []
+    for _ in range(6):
+        out.append(i)
+        i += 1 + 2 * int(flat[i])
+    return out
+
+
+def with_map(flat, dof, which, entries):
+    a = maps_at(flat, dof)[which]
+    b = a + 1 + 2 * int(flat[a])
+    e = np.asarray(entries, dtype=np.float64)
+    return np.concatenate([flat[:a], [len(e)], e.ravel(), flat[b:]])
+
+
+def map_of(flat, dof, which):
+    a = maps_at(flat, dof)[which]
+    return flat[a + 1:a + 1 + 2 * int(flat[a])].reshape(-1, 2).copy()
+
+
+def inputs(dof, nr, flat, seed):
+    """Moving and resting vehicles, steering both ways, throttle and braking, own parameters; one vehicle
+    light enough to lift wheels."""
+    rng = np.random.Generator(np.random.PCG64(seed))
+    recs = W.initial_speed_records(N, flat, dof, seed=seed, umax=25.0, tire_nr=nr)
+    recs[0] = 0.0
+    ovr = W.knot_fleet(N, flat, seed=seed, dof=dof, tire_nr=nr)["ovr"]
+    ovr[0, 1] *= 0.3
+    ovr[5] = rng.uniform(0.5, 1.5, N)
+    if dof == 24:
+        recs = O.init24(flat, recs, nr, ovr)
+    t = np.arange(STEPS)[:, None] * 1e-3
+    ctrl = np.empty((STEPS, 3, N))
+    ctrl[:, 0] = rng.uniform(0.2, 1.0, N) * np.sin(2 * np.pi * rng.uniform(1, 6, N) * t + rng.uniform(0, 6.3, N))
+    ctrl[:, 1] = rng.uniform(0, 1, (STEPS // 50, N)).repeat(50, axis=0)
+    ctrl[:, 2] = np.where(rng.random((STEPS // 50, N)) < 0.3, 0.6, 0.0).repeat(50, axis=0)
+    return np.ascontiguousarray(recs), np.ascontiguousarray(ovr), np.ascontiguousarray(ctrl)
+
+
+def run(dof, nr, lanes, flat, recs, ovr, ctrl):
+    assert os.path.exists(LIB), "run make -C low-fidelity-dynamic-models_amd groupstep"
+    L = ctypes.CDLL(LIB)
+    i, p, d = ctypes.c_int, ctypes.c_void_p, ctypes.c_double
+    L.group_step_run.argtypes = [i, i, i, p, i, p, p, i, i, i, p, d, p, p]
+    flat = np.ascontiguousarray(flat)
+    fin, walks = np.zeros_like(recs), ctypes.c_int()
+    assert L.group_step_run(dof, int(nr), lanes, flat.ctypes.data, flat.size, ovr.ctypes.data, recs.ctypes.data,
+                            recs.shape[0], recs.shape[1], ctrl.shape[0], ctrl.ctypes.data, 1e-3, fin.ctypes.data,
+                            ctypes.byref(walks)) == 0
+    return fin, walks.value
+
+
+def check(dof, nr, flat, seed, walks):
+    recs, ovr, ctrl = inputs(dof, nr, flat, seed)
+    for steps in (STEPS, 1):
+        c = np.ascontiguousarray(ctrl[:steps])
+        ref, _ = run(dof, nr, 1, flat, recs, ovr, c)
+        assert np.isfinite(ref).all() and not np.array_equal(ref, recs)
+        for lanes in (2,) if dof == 11 else (2, 4):
+            got, w = run(dof, nr, lanes, flat, recs, ovr, c)
+            np.testing.assert_array_equal(got, ref, err_msg=f"{dof}-DOF, {lanes} lanes, {steps} steps")
+            assert w == int(walks)
+
+
+VEHICLES = [  # vehicle, tire, TMeasyNr?, served by the walk
+    ("HMMWV/vehicle.json", "HMMWV/tmeasy.json", False, True),
+    ("Sedan/vehicle.json", "Sedan/tmeasyNr.json", True, True),
+    ("Sedan/vehicle_RWD.json", "Sedan/tmeasy.json", False, True),
+    ("audi/vehicle.json", "audi/tmeasy.json", False, True),
+    ("ART/vehicle.json", "ART/tmeasy.json", False, False),
+]
+
+
+CASES = [(dof, *v) for v in VEHICLES for dof in (11, 18, 24) if dof < 24 or v[0] in [VEHICLES[0][0], VEHICLES[1][0]]]
+
+
+@pytest.mark.parametrize("dof,veh,tire,nr,walks", CASES, ids=[f"{c[0]}-{c[1]}-{c[2]}" for c in CASES])
+def test_group_step_gives_the_one_lane_bits(dof, veh, tire, nr, walks):
+    check(dof, nr, params(dof, veh, tire, nr), 21 + dof, walks)
+
+
+@pytest.mark.parametrize("dof", [11, 18, 24])
+@pytest.mark.parametrize("form", ["front_drive", "one_entry", "equal_knots", "full_table", "not_ascending"])
+def test_group_step_on_other_powertrains(dof, form):
+    """Front drive; a losses map of one entry; maps with equal neighbouring abscissae; a torque map of all 48
+    entries (several knots passed in one step); a map that does not ascend, which the walk leaves to the scan."""
+    flat = params(dof, "HMMWV/vehicle.json", "HMMWV/tmeasy.json", False)
+    torque = map_of(flat, dof, 2)
+    walks = True
+    if form == "front_drive":
+        flat[W.FLAT[dof]["gears"] - 2:W.FLAT[dof]["gears"]] = 0.0
+    elif form == "one_entry":
+        flat = with_map(flat, dof, 3, [[100.0, -12.0]])
+    elif form == "equal_knots":
+        torque[5, 0] = torque[4, 0]
+        cf = map_of(flat, dof, 4)
+        cf[2, 0] = cf[1, 0]
+        flat = with_map(with_map(flat, dof, 2, torque), dof, 4, cf)
+    elif form == "full_table":
+        x = np.linspace(torque[0, 0], torque[-1, 0], 48)
+        flat = with_map(flat, dof, 2, np.stack([x, np.interp(x, torque[:, 0], torque[:, 1])], 1))
+    else:
+        torque[[3, 6]] = torque[[6, 3]]
+        flat = with_map(flat, dof, 2, torque)
+        walks = False
+    check(dof, False, flat, 5 + dof, walks)
