@@ -516,6 +516,140 @@ LFDM_HD void powertrain4_adj(const PSet& P, const Derived& u, double tqs, double
     }
 }
 
+// The chassis part of the step's adjoint, shared by the one-lane and the lane-group form: forward recompute
+// of the accelerations from the tire forces gfx, gfy in the vehicle's axes, then the adjoints of the
+// position and velocity updates and of computeVehRHS.  S: a state's chassis fields before the step; o, sb:
+// the adjoints after and before it (sb accumulates); sp, cp: sine and cosine of the yaw angle.
+template <class S, class B>
+LFDM_HD void chassis18_adj(const PSet& P, const Derived& u, const K18& k, const S& s0, const double* gfx,
+                           const double* gfy, double sp, double cp, double dt, const B& o, B& sb, K18b& kb,
+                           double* gfxb, double* gfyb) {
+    const double jxz = P.jxz, jz = k.jz, A1 = u.A1, A2 = k.A2, A3 = k.A3, mt = -k.neg_mt;
+    const double E1 = k.neg_mt * s0.wz * s0.u + (gfy[0] + gfy[1] + gfy[2] + gfy[3]);
+    const double E2 = (gfy[0] + gfy[1]) * P.a - (gfy[2] + gfy[3]) * P.b + (gfx[1] - gfx[0]) * P.cf / 2 +
+                      (gfx[3] - gfx[2]) * P.cr / 2 + u.E2c * s0.wz * s0.u;
+    const double E3 = k.E3c * s0.phi - u.kro * s0.phi - u.bro * s0.wx + k.hm * s0.wz * s0.u;
+    const double inner = (gfx[0] + gfx[1] + gfx[2] + gfx[3]) + u.Uc * (s0.wz * s0.wz) - k.two_hrc_m * s0.wz * s0.wx;
+    const double vdot = (E1 * u.jxz2 - k.A1A2 * E2 + A1 * E3 * jxz + A3 * E2 * jxz - A2 * E1 * jz - A3 * E3 * jz) *
+                        k.rdenom;
+    const double wxdot =
+        (u.A1sq * E3 - k.A1A3 * E2 + A1 * E1 * jxz - A3 * E1 * jz + E2 * jxz * mt - E3 * jz * mt) * k.rdenom;
+    const double wzdot =
+        (k.A3sq * E2 - k.A1A2 * E1 - k.A1A3 * E3 + A3 * E1 * jxz - A2 * E2 * mt + E3 * jxz * mt) * k.rdenom;
+    const double udot = s0.wz * s0.v + k.inv_mt * inner;
+    const double un = s0.u + udot * dt, vn = s0.v + vdot * dt;
+    // x' = x + (u' cp - v' sp) dt, y' = y + (u' sp + v' cp) dt
+    double unb = o.u, vnb = o.v, wznb = o.wz, wxnb = o.wx;
+    sb.x += o.x;
+    sb.y += o.y;
+    unb += o.x * cp * dt + o.y * sp * dt;
+    vnb += -o.x * sp * dt + o.y * cp * dt;
+    sb.psi += o.x * (-un * sp - vn * cp) * dt + o.y * (un * cp - vn * sp) * dt;
+    // psi' = psi + wz' dt, phi' = phi + wx' dt
+    sb.psi += o.psi;
+    wznb += o.psi * dt;
+    sb.phi += o.phi;
+    wxnb += o.phi * dt;
+    // u' = u + udot dt (and udot' = udot), likewise v, wx, wz
+    sb.u += unb;
+    double udotb = unb * dt + o.udot;
+    sb.v += vnb;
+    double vdotb = vnb * dt + o.vdot;
+    sb.wx += wxnb;
+    const double wxdotb = wxnb * dt;
+    sb.wz += wznb;
+    const double wzdotb = wznb * dt;
+    // ---- chassis (computeVehRHS) ----
+    const double rden = k.rdenom;
+    const double Nvb = vdotb * rden, Nxb = wxdotb * rden, Nzb = wzdotb * rden;
+    kb.denom -= (Nvb * vdot + Nxb * wxdot + Nzb * wzdot);
+    double E1b = Nvb * (u.jxz2 - A2 * jz) + Nxb * (A1 * jxz - A3 * jz) + Nzb * (-k.A1A2 + A3 * jxz);
+    double E2b = Nvb * (-k.A1A2 + A3 * jxz) + Nxb * (-k.A1A3 + jxz * mt) + Nzb * (k.A3sq - A2 * mt);
+    double E3b = Nvb * (A1 * jxz - A3 * jz) + Nxb * (u.A1sq - jz * mt) + Nzb * (-k.A1A3 + jxz * mt);
+    kb.A1A2 -= Nvb * E2 + Nzb * E1;
+    kb.A1A3 -= Nxb * E2 + Nzb * E3;
+    kb.A3sq += Nzb * E2;
+    kb.A3 += Nvb * (E2 * jxz - E3 * jz) - Nxb * E1 * jz + Nzb * jxz * E1;
+    kb.A2 -= Nvb * E1 * jz + Nzb * mt * E2;
+    kb.jz -= Nvb * (A2 * E1 + A3 * E3) + Nxb * (A3 * E1 + mt * E3);
+    const double mtb = Nxb * (jxz * E2 - jz * E3) + Nzb * (-A2 * E2 + jxz * E3);
+    kb.neg_mt -= mtb;
+    // udot = wz v + inv_mt inner
+    sb.v += udotb * s0.wz;
+    sb.wz += udotb * s0.v;
+    kb.inv_mt += udotb * inner;
+    const double innerb = udotb * k.inv_mt;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+        gfxb[i] = innerb;
+        gfyb[i] = E1b;
+    }
+    sb.wz += innerb * (2.0 * u.Uc * s0.wz - k.two_hrc_m * s0.wx);
+    sb.wx -= innerb * k.two_hrc_m * s0.wz;
+    kb.two_hrc_m -= innerb * s0.wz * s0.wx;
+    // E1 = neg_mt wz u + sum fy
+    kb.neg_mt += E1b * s0.wz * s0.u;
+    sb.wz += E1b * k.neg_mt * s0.u;
+    sb.u += E1b * k.neg_mt * s0.wz;
+    // E2
+    gfyb[0] += E2b * P.a;
+    gfyb[1] += E2b * P.a;
+    gfyb[2] -= E2b * P.b;
+    gfyb[3] -= E2b * P.b;
+    gfxb[1] += E2b * P.cf / 2;
+    gfxb[0] -= E2b * P.cf / 2;
+    gfxb[3] += E2b * P.cr / 2;
+    gfxb[2] -= E2b * P.cr / 2;
+    sb.wz += E2b * u.E2c * s0.u;
+    sb.u += E2b * u.E2c * s0.wz;
+    // E3
+    kb.E3c += E3b * s0.phi;
+    sb.phi += E3b * (k.E3c - u.kro);
+    sb.wx -= E3b * u.bro;
+    kb.hm += E3b * s0.wz * s0.u;
+    sb.wz += E3b * k.hm * s0.u;
+    sb.u += E3b * k.hm * s0.wz;
+}
+
+// The adjoint of the steering angle and the contact-patch velocities (vehToTireTransform) and of
+// computeTireLoads, from the tires' bars: vsxb, vsyb, rb (the loads', zero for a clamped load), deltab (the
+// slip angles'), sdb and cdb (the force rotation's).
+template <class S, class B>
+LFDM_HD void body18_adj(const PSet& P, const Derived& u, const K18& k, const S& s0, double lat, double sd, double cd,
+                        double vsy0, const double* vsxb, const double* vsyb, const double* rb, double deltab,
+                        double sdb, double cdb, B& sb, double& steerb, K18b& kb) {
+    // ---- vehToTireTransform ----
+    const double m0b = vsxb[0] * cd, m1b = vsxb[1] * cd;
+    cdb += vsxb[0] * (s0.u - (s0.wz * P.cf) / 2.) + vsxb[1] * (s0.u + (s0.wz * P.cf) / 2.);
+    sdb += (vsxb[0] + vsxb[1]) * vsy0;
+    const double vsy0b = vsyb[0] + vsyb[1] + (vsxb[0] + vsxb[1]) * sd;
+    sb.u += m0b + m1b + vsxb[2] + vsxb[3];
+    sb.wz += (m1b - m0b) * P.cf / 2. + (vsxb[3] - vsxb[2]) * P.cr / 2.;
+    sb.v += vsy0b + vsyb[2] + vsyb[3];
+    sb.wz += vsy0b * P.a - (vsyb[2] + vsyb[3]) * P.b;
+    deltab += sdb * cd - cdb * sd;
+    steerb += deltab * P.maxSteer;
+    // ---- computeTireLoads ----
+    kb.Z1f += rb[0] + rb[1];
+    kb.Z1r += rb[2] + rb[3];
+    const double Z2fb = -rb[0] + rb[1], Z3fb = -rb[0] + rb[1];
+    const double Z2rb = -rb[2] + rb[3], Z3rb = -rb[2] + rb[3];
+    const double Z4b = -rb[0] - rb[1] + rb[2] + rb[3];
+    kb.Z2fc += Z2fb * lat;
+    kb.Z2rc += Z2rb * lat;
+    const double latb = Z2fb * k.Z2fc + Z2rb * k.Z2rc;
+    sb.phi += Z3fb * u.krof_cf + Z3rb * u.kror_cr;
+    sb.wx += Z3fb * u.brof_cf + Z3rb * u.bror_cr;
+    kb.Z4n += Z4b * (s0.udot - s0.wz * s0.v) * u.inv_two_ab;
+    const double ddb = Z4b * k.Z4n * u.inv_two_ab;
+    sb.udot += ddb;
+    sb.wz -= ddb * s0.v;
+    sb.v -= ddb * s0.wz;
+    sb.vdot += latb;
+    sb.wz += latb * s0.u;
+    sb.u += latb * s0.wz;
+}
+
 // Adjoint of one half-implicit step.  s0: state before the step (gear included); sb: in = adjoint
 // of the state after the step, out = adjoint of the state before it; controls' bars are returned,
 // constants' bars accumulated into kb.
@@ -578,10 +712,6 @@ LFDM_HD void step18_adj(const PSet& P, const Derived& u, const K18& k, const S18
                         xedot[i], yedot[i], om[i], fx[i], fy[i], My[i], xt, rStat[i]);
         }
     }
-    double crank = s0.crank;
-    int gear = s0.gear;
-    double dOm[4], eng[4], dcrank;
-    powertrain4<false>(P, u, k.tqs, k.maxBrake, throttle, braking, s0.u, crank, gear, om, fx, rStat, My, dOm, eng, dcrank);
     double gfx[4], gfy[4];
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
@@ -593,47 +723,12 @@ LFDM_HD void step18_adj(const PSet& P, const Derived& u, const K18& k, const S18
         gfx[i] = fx[i] * cd - fy[i] * sd;
         gfy[i] = fx[i] * sd + fy[i] * cd;
     }
-    const double jxz = P.jxz, jz = k.jz, A1 = u.A1, A2 = k.A2, A3 = k.A3, mt = -k.neg_mt;
-    const double E1 = k.neg_mt * s0.wz * s0.u + (gfy[0] + gfy[1] + gfy[2] + gfy[3]);
-    const double E2 = (gfy[0] + gfy[1]) * P.a - (gfy[2] + gfy[3]) * P.b + (gfx[1] - gfx[0]) * P.cf / 2 +
-                      (gfx[3] - gfx[2]) * P.cr / 2 + u.E2c * s0.wz * s0.u;
-    const double E3 = k.E3c * s0.phi - u.kro * s0.phi - u.bro * s0.wx + k.hm * s0.wz * s0.u;
-    const double inner = (gfx[0] + gfx[1] + gfx[2] + gfx[3]) + u.Uc * (s0.wz * s0.wz) - k.two_hrc_m * s0.wz * s0.wx;
-    const double vdot = (E1 * u.jxz2 - k.A1A2 * E2 + A1 * E3 * jxz + A3 * E2 * jxz - A2 * E1 * jz - A3 * E3 * jz) *
-                        k.rdenom;
-    const double wxdot =
-        (u.A1sq * E3 - k.A1A3 * E2 + A1 * E1 * jxz - A3 * E1 * jz + E2 * jxz * mt - E3 * jz * mt) * k.rdenom;
-    const double wzdot =
-        (k.A3sq * E2 - k.A1A2 * E1 - k.A1A3 * E3 + A3 * E1 * jxz - A2 * E2 * mt + E3 * jxz * mt) * k.rdenom;
-    const double udot = s0.wz * s0.v + k.inv_mt * inner;
-    const double un = s0.u + udot * dt, vn = s0.v + vdot * dt, wzn = s0.wz + wzdot * dt;
     double sp, cp;
     sincos_fast(s0.psi, sp, cp);
 
     // ================= reverse =================
     S18b o = sb;  // bars of the state after the step
     s18b_zero(sb);
-    // x' = x + (u' cp - v' sp) dt, y' = y + (u' sp + v' cp) dt
-    double unb = o.u, vnb = o.v, wznb = o.wz, wxnb = o.wx;
-    sb.x += o.x;
-    sb.y += o.y;
-    unb += o.x * cp * dt + o.y * sp * dt;
-    vnb += -o.x * sp * dt + o.y * cp * dt;
-    sb.psi += o.x * (-un * sp - vn * cp) * dt + o.y * (un * cp - vn * sp) * dt;
-    // psi' = psi + wz' dt, phi' = phi + wx' dt
-    sb.psi += o.psi;
-    wznb += o.psi * dt;
-    sb.phi += o.phi;
-    wxnb += o.phi * dt;
-    // u' = u + udot dt (and udot' = udot), likewise v, wx, wz
-    sb.u += unb;
-    double udotb = unb * dt + o.udot;
-    sb.v += vnb;
-    double vdotb = vnb * dt + o.vdot;
-    sb.wx += wxnb;
-    const double wxdotb = wxnb * dt;
-    sb.wz += wznb;
-    const double wzdotb = wznb * dt;
     // crank' = crank + dcrank dt (converter) or the slaved crank
     PtBars pb;
 #pragma unroll
@@ -664,57 +759,8 @@ LFDM_HD void step18_adj(const PSet& P, const Derived& u, const K18& k, const S18
         yedotb[i] = o.ye[i] * dt + o.yedot[i];
         omb[i] = o.omega[i];
     }
-    // ---- chassis (computeVehRHS) ----
-    const double rden = k.rdenom;
-    const double Nvb = vdotb * rden, Nxb = wxdotb * rden, Nzb = wzdotb * rden;
-    kb.denom -= (Nvb * vdot + Nxb * wxdot + Nzb * wzdot);
-    double E1b = Nvb * (u.jxz2 - A2 * jz) + Nxb * (A1 * jxz - A3 * jz) + Nzb * (-k.A1A2 + A3 * jxz);
-    double E2b = Nvb * (-k.A1A2 + A3 * jxz) + Nxb * (-k.A1A3 + jxz * mt) + Nzb * (k.A3sq - A2 * mt);
-    double E3b = Nvb * (A1 * jxz - A3 * jz) + Nxb * (u.A1sq - jz * mt) + Nzb * (-k.A1A3 + jxz * mt);
-    kb.A1A2 -= Nvb * E2 + Nzb * E1;
-    kb.A1A3 -= Nxb * E2 + Nzb * E3;
-    kb.A3sq += Nzb * E2;
-    kb.A3 += Nvb * (E2 * jxz - E3 * jz) - Nxb * E1 * jz + Nzb * jxz * E1;
-    kb.A2 -= Nvb * E1 * jz + Nzb * mt * E2;
-    kb.jz -= Nvb * (A2 * E1 + A3 * E3) + Nxb * (A3 * E1 + mt * E3);
-    const double mtb = Nxb * (jxz * E2 - jz * E3) + Nzb * (-A2 * E2 + jxz * E3);
-    kb.neg_mt -= mtb;
-    // udot = wz v + inv_mt inner
-    sb.v += udotb * s0.wz;
-    sb.wz += udotb * s0.v;
-    kb.inv_mt += udotb * inner;
-    const double innerb = udotb * k.inv_mt;
     double gfxb[4], gfyb[4];
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-        gfxb[i] = innerb;
-        gfyb[i] = E1b;
-    }
-    sb.wz += innerb * (2.0 * u.Uc * s0.wz - k.two_hrc_m * s0.wx);
-    sb.wx -= innerb * k.two_hrc_m * s0.wz;
-    kb.two_hrc_m -= innerb * s0.wz * s0.wx;
-    // E1 = neg_mt wz u + sum fy
-    kb.neg_mt += E1b * s0.wz * s0.u;
-    sb.wz += E1b * k.neg_mt * s0.u;
-    sb.u += E1b * k.neg_mt * s0.wz;
-    // E2
-    gfyb[0] += E2b * P.a;
-    gfyb[1] += E2b * P.a;
-    gfyb[2] -= E2b * P.b;
-    gfyb[3] -= E2b * P.b;
-    gfxb[1] += E2b * P.cf / 2;
-    gfxb[0] -= E2b * P.cf / 2;
-    gfxb[3] += E2b * P.cr / 2;
-    gfxb[2] -= E2b * P.cr / 2;
-    sb.wz += E2b * u.E2c * s0.u;
-    sb.u += E2b * u.E2c * s0.wz;
-    // E3
-    kb.E3c += E3b * s0.phi;
-    sb.phi += E3b * (k.E3c - u.kro);
-    sb.wx -= E3b * u.bro;
-    kb.hm += E3b * s0.wz * s0.u;
-    sb.wz += E3b * k.hm * s0.u;
-    sb.u += E3b * k.hm * s0.wz;
+    chassis18_adj(P, u, k, s0, gfx, gfy, sp, cp, dt, o, sb, kb, gfxb, gfyb);
     // ---- tireToVehTransform (front tires rotated by delta) ----
     double fxb[4], fyb[4];
     double sdb = 0, cdb = 0;
@@ -772,39 +818,11 @@ LFDM_HD void step18_adj(const PSet& P, const Derived& u, const K18& k, const S18
         kb.qy1 += tb.qy1;
         kb.qy2 += tb.qy2;
     }
-    // ---- vehToTireTransform ----
-    const double m0b = vsxb[0] * cd, m1b = vsxb[1] * cd;
-    cdb += vsxb[0] * (s0.u - (s0.wz * P.cf) / 2.) + vsxb[1] * (s0.u + (s0.wz * P.cf) / 2.);
-    sdb += (vsxb[0] + vsxb[1]) * vsy[0];
-    const double vsy0b = vsyb[0] + vsyb[1] + (vsxb[0] + vsxb[1]) * sd;
-    sb.u += m0b + m1b + vsxb[2] + vsxb[3];
-    sb.wz += (m1b - m0b) * P.cf / 2. + (vsxb[3] - vsxb[2]) * P.cr / 2.;
-    sb.v += vsy0b + vsyb[2] + vsyb[3];
-    sb.wz += vsy0b * P.a - (vsyb[2] + vsyb[3]) * P.b;
-    deltab += sdb * cd - cdb * sd;
-    steerb += deltab * P.maxSteer;
-    // ---- computeTireLoads ----
+    // ---- vehToTireTransform, computeTireLoads ----
     double rb[4];
 #pragma unroll
     for (int i = 0; i < 4; ++i) rb[i] = fzr[i] > 0. ? fzb[i] : 0.;
-    kb.Z1f += rb[0] + rb[1];
-    kb.Z1r += rb[2] + rb[3];
-    const double Z2fb = -rb[0] + rb[1], Z3fb = -rb[0] + rb[1];
-    const double Z2rb = -rb[2] + rb[3], Z3rb = -rb[2] + rb[3];
-    const double Z4b = -rb[0] - rb[1] + rb[2] + rb[3];
-    kb.Z2fc += Z2fb * lat;
-    kb.Z2rc += Z2rb * lat;
-    const double latb = Z2fb * k.Z2fc + Z2rb * k.Z2rc;
-    sb.phi += Z3fb * u.krof_cf + Z3rb * u.kror_cr;
-    sb.wx += Z3fb * u.brof_cf + Z3rb * u.bror_cr;
-    kb.Z4n += Z4b * (s0.udot - s0.wz * s0.v) * u.inv_two_ab;
-    const double ddb = Z4b * k.Z4n * u.inv_two_ab;
-    sb.udot += ddb;
-    sb.wz -= ddb * s0.v;
-    sb.v -= ddb * s0.wz;
-    sb.vdot += latb;
-    sb.wz += latb * s0.u;
-    sb.u += latb * s0.wz;
+    body18_adj(P, u, k, s0, lat, sd, cd, vsy[0], vsxb, vsyb, rb, deltab, sdb, cdb, sb, steerb, kb);
 }
 
 // Adjoint of k18_init: bars of the per-vehicle parameters (m, jz, jx, dfy0Pn, dfy0P2n, tqs, maxBrake)

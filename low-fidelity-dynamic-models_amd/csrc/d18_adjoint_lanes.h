@@ -170,6 +170,16 @@ LFDM_HD void adj_forward_lane(const AdjLaunch& L, int slot, const PSet& P) {
 constexpr int kCarry = 31 + 21;
 static_assert(kCarried == kAdjCkptRow && kSegRow == kAdjTapeRow && kCarry == kAdjCarry, "adjoint buffer rows");
 
+// The rows of the chassis's adjoints and the constants'.
+LFDM_HD void store_carry_body(const S18b& l, const K18b& kb, double* p, size_t S) {
+    const double v[32] = {l.x,      l.y,       l.u,     l.v,         l.psi,    l.wz,    l.phi,    l.wx,
+                          l.udot,   l.vdot,    l.crank, kb.Z1f,      kb.Z2fc,  kb.Z1r,  kb.Z2rc,  kb.Z4n,
+                          kb.neg_mt, kb.E3c,   kb.hm,   kb.A2,       kb.A3,    kb.inv_mt, kb.two_hrc_m, kb.denom,
+                          kb.A1A2,  kb.A1A3,   kb.A3sq, kb.qy1,      kb.qy2,   kb.jz,   kb.tqs,   kb.maxBrake};
+#pragma unroll
+    for (int j = 0; j < 32; ++j) p[(20 + j) * S] = v[j];
+}
+
 LFDM_HD void store_carry(const S18b& l, const K18b& kb, double* p, size_t S) {
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
@@ -179,12 +189,7 @@ LFDM_HD void store_carry(const S18b& l, const K18b& kb, double* p, size_t S) {
         p[(12 + i) * S] = l.yedot[i];
         p[(16 + i) * S] = l.omega[i];
     }
-    const double v[32] = {l.x,      l.y,       l.u,     l.v,         l.psi,    l.wz,    l.phi,    l.wx,
-                          l.udot,   l.vdot,    l.crank, kb.Z1f,      kb.Z2fc,  kb.Z1r,  kb.Z2rc,  kb.Z4n,
-                          kb.neg_mt, kb.E3c,   kb.hm,   kb.A2,       kb.A3,    kb.inv_mt, kb.two_hrc_m, kb.denom,
-                          kb.A1A2,  kb.A1A3,   kb.A3sq, kb.qy1,      kb.qy2,   kb.jz,   kb.tqs,   kb.maxBrake};
-#pragma unroll
-    for (int j = 0; j < 32; ++j) p[(20 + j) * S] = v[j];
+    store_carry_body(l, kb, p, S);
 }
 
 LFDM_HD void load_carry(const double* p, size_t S, S18b& l, K18b& kb) {

@@ -19,19 +19,17 @@ struct S18g {
     GearRow row;
 };
 
-// Per-vehicle constants, and those of this lane's axle or tire: with a tire per lane the load
+// Constants of this lane's axle or tire (beside the vehicle's K18): with a tire per lane the load
 // transfers and the half track carry its side's sign (negation is exact), so that one expression
 // serves all four.
 template <int G>
 struct K18g {
-    K18 c;
     bool front, walks;
     double Z1, Z2c, kro, bro, inv_c, inv_two_ab, track, arm;
 };
 
 template <int G>
 LFDM_HD void k18g_init(const PSet& P, const K18& c, int q, K18g<G>& k) {
-    k.c = c;
     k.front = G == 4 ? q < 2 : q == 0;
     k.walks = group_walks(P);
     const double side = G == 4 && (q & 1) == 0 ? -1.0 : 1.0;  // a left tire's lane: minus
@@ -61,30 +59,63 @@ LFDM_HD void move18g(S18g<G>& s, double sp, double cp, double dt) {
     s.psi = s.psi + s.wz * dt;
 }
 
-// step18 without its closing position update; `lag`: the previous step's position update comes first
-// (its sine and cosine of the yaw angle from one lane while another takes the steering angle's).
-template <bool NR, bool FULL, int G>
-LFDM_HD void step18g(const PSet& P, const Derived& u, const K18g<G>& k, S18g<G>& s, double steering, double throttle,
-                     double braking, double dt, bool lag, X18g<G>* x) {
-    constexpr int N = 4 / G;
-    const TireP& t = P.tire;
+// The step's steering angle, with the previous step's position update (`lag`): one lane takes the sine and
+// cosine of the steering angle while another takes the yaw angle's.
+template <int G>
+LFDM_HD void angles18g(const PSet& P, S18g<G>& s, double steering, double dt, bool lag, double& sd, double& cd) {
     const double delta = P.nonLinearSteer ? map_y<false>(P.steer, steering) : steering * P.maxSteer;
     double sa, ca;
     sincos_fast((s.q & 1) ? s.psi : delta, sa, ca);
-    const double sd = group_value<G, 0>(sa), cd = group_value<G, 0>(ca);
+    sd = group_value<G, 0>(sa);
+    cd = group_value<G, 0>(ca);
     if (lag) move18g<G>(s, group_value<G, 1>(sa), group_value<G, 1>(ca), dt);
-    // computeTireLoads
-    const double lat = s.vdot + s.wz * s.u;
+}
+
+// A lane's tire right-hand-side outputs of one step (before the front forces are rotated), for the tape.
+template <int G>
+struct TireOut18g {
+    static constexpr int N = 4 / G;
+    double fx[N], fy[N], My[N], rStat[N];
+};
+
+// This lane's wheel loads, before the clamp at zero.
+template <int G>
+LFDM_HD void loads18g(const K18& c, const K18g<G>& k, double lat, double phi, double wx, double udot, double wz, double v,
+                      double* fz) {
     const double Z2 = k.Z2c * lat;
-    const double Z3 = (k.kro * s.phi + k.bro * s.wx) * k.inv_c;
-    const double Z4 = (k.c.Z4n * (s.udot - s.wz * s.v)) * k.inv_two_ab;
-    double fz[N];
+    const double Z3 = (k.kro * phi + k.bro * wx) * k.inv_c;
+    const double Z4 = (c.Z4n * (udot - wz * v)) * k.inv_two_ab;
     if constexpr (G == 4) {
         fz[0] = k.Z1 + Z2 + Z3 + Z4;
     } else {
         fz[0] = k.Z1 - Z2 - Z3 + Z4;
         fz[1] = k.Z1 + Z2 + Z3 + Z4;
     }
+}
+
+// This lane's contact-patch velocities; returns the lateral one, the longitudinal ones in vsx.
+template <int G>
+LFDM_HD double patch18g(const K18g<G>& k, double u, double v, double wz, double sd, double cd, double* vsx) {
+    const double vsy = v + wz * k.arm;
+    const double hw = (wz * k.track) / 2.;
+#pragma unroll
+    for (int j = 0; j < 4 / G; ++j) {
+        const double vx = G == 4 || j == 1 ? u + hw : u - hw;
+        const double vf = vx * cd + vsy * sd;
+        vsx[j] = k.front ? vf : vx;
+    }
+    return vsy;
+}
+
+// step18 without its closing position update, after angles18g.
+template <bool NR, bool FULL, int G, bool CAPTURE = false>
+LFDM_HD void step18g(const PSet& P, const Derived& u, const K18& c, const K18g<G>& k, S18g<G>& s, double sd, double cd,
+                     double throttle, double braking, double dt, X18g<G>* x, TireOut18g<G>* to = nullptr) {
+    constexpr int N = 4 / G;
+    const TireP& t = P.tire;
+    // computeTireLoads
+    double fz[N];
+    loads18g<G>(c, k, s.vdot + s.wz * s.u, s.phi, s.wx, s.udot, s.wz, s.v, fz);
 #pragma unroll
     for (int j = 0; j < N; ++j) fz[j] = fz[j] > 0. ? fz[j] : 0.;
     // wheel speeds as the powertrain will read them: a tire off the ground resets its own (tire_tmeasy)
@@ -95,7 +126,7 @@ LFDM_HD void step18g(const PSet& P, const Derived& u, const K18g<G>& k, S18g<G>&
     // the powertrain's torque: nothing in it depends on this step's tire forces, so it comes first and
     // its dependent chain overlaps the tire's
     double shaft, dcrank;
-    powertrain_group<G>(P, u, k.c.tqs, throttle, s.u, 0.25 * (om4[0] + om4[1] + om4[2] + om4[3]), s.q, k.walks, s.maps,
+    powertrain_group<G>(P, u, c.tqs, throttle, s.u, 0.25 * (om4[0] + om4[1] + om4[2] + om4[3]), s.q, k.walks, s.maps,
                         s.row, s.crank, s.gear, shaft, dcrank);
     double tf, tr;
     axle_torques(P, shaft, tf, tr);
@@ -111,15 +142,8 @@ LFDM_HD void step18g(const PSet& P, const Derived& u, const K18g<G>& k, S18g<G>&
         }
     }
     // vehToTireTransform
-    const double vsy = s.v + s.wz * k.arm;
-    const double hw = (s.wz * k.track) / 2.;
     double vsx[N];
-#pragma unroll
-    for (int j = 0; j < N; ++j) {
-        const double vx = G == 4 || j == 1 ? s.u + hw : s.u - hw;
-        const double vf = vx * cd + vsy * sd;
-        vsx[j] = k.front ? vf : vx;
-    }
+    const double vsy = patch18g<G>(k, s.u, s.v, s.wz, sd, cd, vsx);
     // computeTireRHS
     const double tand = fdiv(sd, cd);
     const double d = k.front ? tand : u.tan_delta_rear;
@@ -127,13 +151,19 @@ LFDM_HD void step18g(const PSet& P, const Derived& u, const K18g<G>& k, S18g<G>&
 #pragma unroll
     for (int j = 0; j < N; ++j) {
         if (!NR)
-            tire_tmeasy<false>(t, u, k.c, 0.0, d, fz[j], vsx[j], vsy, s.xe[j], s.ye[j], s.xedot[j], s.yedot[j],
+            tire_tmeasy<false>(t, u, c, 0.0, d, fz[j], vsx[j], vsy, s.xe[j], s.ye[j], s.xedot[j], s.yedot[j],
                                s.omega[j], fx[j], fy[j], My[j], xt[j], rStat[j]);
         else
-            tire_tmeasy_nr<false>(t, u, k.c, 0.0, d, fz[j], vsx[j], vsy, s.omega[j], fx[j], fy[j], My[j], xt[j],
+            tire_tmeasy_nr<false>(t, u, c, 0.0, d, fz[j], vsx[j], vsy, s.omega[j], fx[j], fy[j], My[j], xt[j],
                                   rStat[j]);
     }
-    const double bt = k.c.maxBrake * braking;
+    if (CAPTURE) {
+#pragma unroll
+        for (int j = 0; j < N; ++j) {
+            to->fx[j] = fx[j]; to->fy[j] = fy[j]; to->My[j] = My[j]; to->rStat[j] = rStat[j];
+        }
+    }
+    const double bt = c.maxBrake * braking;
     double dOm[N];
 #pragma unroll
     for (int j = 0; j < N; ++j) dOm[j] = u.inv_jw * (eng[j] + My[j] - sgn(s.omega[j]) * bt - fx[j] * rStat[j]);
@@ -149,7 +179,7 @@ LFDM_HD void step18g(const PSet& P, const Derived& u, const K18g<G>& k, S18g<G>&
     group_tires<G>(fx, fx4);
     group_tires<G>(fy, fy4);
     double udot, vdot, wxdot, wzdot;
-    chassis18<false>(P, u, k.c, s.u, s.v, s.wz, s.wx, s.phi, fx4, fy4, udot, vdot, wxdot, wzdot);
+    chassis18<false>(P, u, c, s.u, s.v, s.wz, s.wx, s.phi, fx4, fy4, udot, vdot, wxdot, wzdot);
 #pragma unroll
     for (int j = 0; j < N; ++j) {
         if (!NR) {

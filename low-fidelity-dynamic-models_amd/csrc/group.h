@@ -83,8 +83,8 @@ LFDM_HD void walk_init(const PSet& P, const MapXY* tab, double tqs, int id, Walk
     w.scale = id == kMapTorque ? tqs : 1.0;
 }
 
-// map_y (map_y_scaled with the ordinates' factor) at x; L, R: the segment of interval w.r.
-LFDM_HD double walk(Walk& w, MapXY L, MapXY R, double x) {
+// Walks to the interval of x; L, R: the segment of interval w.r, before and after.
+LFDM_HD void walk_to(Walk& w, MapXY& L, MapXY& R, double x) {
     for (;;) {
         const bool down = w.r > 1 && !(L.x < x), up = w.r < w.n - 1 && R.x < x;
         if (!(down || up)) break;
@@ -92,6 +92,11 @@ LFDM_HD double walk(Walk& w, MapXY L, MapXY R, double x) {
         L = w.e[w.r - 1];
         R = w.e[w.r];
     }
+}
+
+// map_y (map_y_scaled with the ordinates' factor) at x; L, R: the segment of interval w.r.
+LFDM_HD double walk(Walk& w, MapXY L, MapXY R, double x) {
+    walk_to(w, L, R, x);
     const double ly = L.y * w.scale, ry = R.y * w.scale;
     const double mbar = fdiv(x - L.x, R.x - L.x);
     const double y = ly + mbar * (ry - ly);

@@ -14,7 +14,10 @@ template <int G>
 struct M18g {
     using S = S18g<G>;
     using X = X18g<G>;
-    using K = K18g<G>;
+    struct K {
+        K18 c;
+        K18g<G> g;
+    };
     static constexpr int kCh = M18::kCh;
     static constexpr bool kKInLds = false;  // a lane's registers hold its constants
     static constexpr int kLanes = G;
@@ -42,16 +45,17 @@ struct M18g {
     }
     // o: the vehicle's parameters (stride S_), tab: the wavefront's maps
     static LFDM_HD void kinit(const PSet& P, const double* o, size_t S_, const MapXY* tab, S& s, K& k) {
-        K18 c;
-        M18::kinit(P, o, S_, c);
-        k18g_init<G>(P, c, s.q, k);
-        walks_init<G>(P, tab, c.tqs, s.q, s.maps);
+        M18::kinit(P, o, S_, k.c);
+        k18g_init<G>(P, k.c, s.q, k.g);
+        walks_init<G>(P, tab, k.c.tqs, s.q, s.maps);
         gear_row(P, s.gear, s.row);
     }
     template <bool NR, bool FULL>
     static LFDM_HD void step(const PSet& P, const Derived& u, const K& k, S& s, const Ctl& c, double dt, bool lag,
                              X* x) {
-        step18g<NR, FULL, G>(P, u, k, s, c.s, c.th, c.b, dt, lag, x);
+        double sd, cd;
+        angles18g<G>(P, s, c.s, dt, lag, sd, cd);
+        step18g<NR, FULL, G>(P, u, k.c, k.g, s, sd, cd, c.th, c.b, dt, x);
     }
     template <bool STRICT>
     static LFDM_HD void position(S& s, double dt) {

@@ -52,6 +52,16 @@ inline KernelChoice choose_kernel(int dof, long long S, int simds, bool strict) 
     return {1, per(1) < most ? (int)per(1) : 0};
 }
 
+// Lanes per vehicle of the adjoint's reverse sweep (its forward follows choose_kernel).  Its step holds more
+// registers than two wavefronts per SIMD have (256 per lane would spill 106 on four lanes, 204 on two: 16,384
+// vehicles 13.0 us per step instead of 6.6, 65,536 on two lanes 37 instead of 17.8 on one), so a vehicle gets
+// more lanes only while they make one wavefront per SIMD at most.  Per step (us) on one lane / two / four:
+//   16,384 vehicles 17.0 / 10.1 / 6.6    32,768 17.0 / 10.6 / -    65,536 17.8 / 21.3 (two rounds)
+inline int reverse_lanes(long long S, int simds) {
+    const long long wf = S / kWave;
+    return wf * 4 <= simds ? 4 : wf * 2 <= simds ? 2 : 1;
+}
+
 struct Launch {
     const PSet* sets;       // parameter sets
     const int* wave_set;   // set index of every 64-slot wavefront
@@ -133,6 +143,8 @@ constexpr int kJacCols = kJacRows + 3;
 // waves_per_simd 1 or 2: register budget of the forward kernel (1 when the fleet fills at most one
 // wavefront per SIMD, so the step runs without spills).
 hipError_t launch_adj_forward(const AdjLaunch& L, int waves_per_simd, hipStream_t stream);
+hipError_t launch_adj_forward_group(const AdjLaunch& L, KernelChoice c, hipStream_t stream);
+hipError_t launch_adj_reverse_group(const AdjLaunch& L, int lanes, hipStream_t stream);
 hipError_t launch_adj_recompute(const AdjLaunch& L, hipStream_t stream);
 hipError_t launch_adj_reverse(const AdjLaunch& L, hipStream_t stream);
 // Every vehicle's step Jacobian at its current record under the per-vehicle controls ctrl[3][n_user].

@@ -1402,7 +1402,8 @@ int lfdm_adjoint_forward(lfdm_solver* h, int nsteps, int checkpoint_every, const
     // a fleet of at most one wavefront per SIMD gets the whole register file per lane
     const int waves = (size_t)h->S / kWave <= (size_t)simds ? 1 : 2;
     HIPCHK(hipEventRecord(h->ev0, h->stream));
-    hipError_t e = launch_adj_forward(L, waves, h->stream);
+    const KernelChoice fc = choose_kernel(18, h->S, simds, false);
+    hipError_t e = fc.lanes > 1 ? launch_adj_forward_group(L, fc, h->stream) : launch_adj_forward(L, waves, h->stream);
     if (e != hipSuccess) return fail(LFDM_E_HIP, std::string("adjoint forward launch failed: ") + hipGetErrorString(e));
     HIPCHK(hipEventRecord(h->ev1, h->stream));
     h->timed = true;
@@ -1459,13 +1460,15 @@ int lfdm_adjoint_backward(lfdm_solver* h, const double* dxy_bar, double* dctrl_b
     L.ctrl_bar = dctrl_bar;
     L.state_bar = dstate_bar;
     L.param_bar = dparam_bar;
+    const int lanes = reverse_lanes(h->S, simd_count(h));
     HIPCHK(hipEventRecord(h->ev0, h->stream));
     for (int hi = nseg; hi > 0; hi -= G) {
         L.seg_hi = hi;
         L.seg_lo = std::max(hi - G, 0);
         hipError_t e = hipSuccess;
         if (!(hi == nseg && h->tape_holds_last)) e = launch_adj_recompute(L, h->stream);
-        if (e == hipSuccess) e = launch_adj_reverse(L, h->stream);
+        if (e == hipSuccess)
+            e = lanes > 1 ? launch_adj_reverse_group(L, lanes, h->stream) : launch_adj_reverse(L, h->stream);
         if (e != hipSuccess)
             return fail(LFDM_E_HIP, std::string("adjoint backward launch failed: ") + hipGetErrorString(e));
     }

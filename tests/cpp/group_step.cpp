@@ -8,6 +8,7 @@
 #include <thread>
 #include <vector>
 
+#include "../../low-fidelity-dynamic-models_amd/csrc/d18_group_adjoint.h"
 #include "../../low-fidelity-dynamic-models_amd/csrc/integrate_group.h"
 #include "../../low-fidelity-dynamic-models_amd/csrc/params.h"
 
@@ -128,6 +129,110 @@ void pick_tire(const Run& r, int nr, const double* init, double* fin) {
 }
 
 }  // namespace
+
+namespace {
+
+// body(q, maps) on G lanes that exchange values.
+template <int G, class F>
+void on_lanes(const PSet& P, F body) {
+    std::vector<MapXY> tab(kGroupMapEntries);
+    for (int id = 0; id < kGroupMaps; ++id)
+        for (int e = 0; e < kMaxMap; ++e) tab[id * kMaxMap + e] = group_map(P, id).e[e];
+    Meeting all(G);
+    std::vector<std::thread> lanes;
+    for (int q = 0; q < G; ++q)
+        lanes.emplace_back([&, q] {
+            t_meeting = &all;
+            t_lane = q;
+            host_group_exchange = exchange;
+            body(q, tab.data());
+        });
+    for (std::thread& t : lanes) t.join();
+}
+
+template <int G>
+void adjoint_group(const PSet& P, AdjLaunch L, int nseg, int group) {
+    for (int v = 0; v < L.n_user; ++v)
+        on_lanes<G>(P, [&](int q, const MapXY* tab) { adj_forward_group<G>(L, v, q, P, tab); });
+    for (int hi = nseg; hi > 0; hi -= group) {
+        L.seg_hi = hi;
+        L.seg_lo = hi - group > 0 ? hi - group : 0;
+        for (int v = 0; v < L.n_user; ++v) {
+            if (hi < nseg)
+                for (int q = 0; q < L.seg_hi - L.seg_lo; ++q) {
+                    K18 k;
+                    adj_recompute_lane(L, q, v, P, k);
+                }
+            // a lane's own storage here: the lanes write the same values, but are not in step
+            on_lanes<G>(P, [&](int q, const MapXY* tab) {
+                K18 k;
+                K18b kb;
+                adj_reverse_group<G>(L, v, q, P, tab, k, kb);
+            });
+        }
+    }
+}
+
+void adjoint_lanes(const PSet& P, AdjLaunch L, int nseg, int group) {
+    for (int v = 0; v < L.n_user; ++v) adj_forward_lane(L, v, P);
+    for (int hi = nseg; hi > 0; hi -= group) {
+        L.seg_hi = hi;
+        L.seg_lo = hi - group > 0 ? hi - group : 0;
+        for (int v = 0; v < L.n_user; ++v) {
+            K18 k;
+            K18b kb;
+            if (hi < nseg)
+                for (int q = 0; q < L.seg_hi - L.seg_lo; ++q) adj_recompute_lane(L, q, v, P, k);
+            adj_reverse_lane(L, v, P, k, kb);
+        }
+    }
+}
+
+}  // namespace
+
+// Adjoint forward and backward of n <= 64 18-DOF vehicles on `lanes` lanes each, checkpoints every K steps and
+// `group` segments per backward group: xy[nsteps][2][n], ctrl_bar[nsteps][3][n], state_bar[75][n],
+// param_bar[7][n].
+extern "C" int group_adjoint_run(int lanes, const double* flat, int len, const double* ovr, const double* init, int n,
+                                 int nsteps, int K, int group, const double* ctrl, const double* xy_bar, double* xy,
+                                 double* ctrl_bar, double* state_bar, double* param_bar) {
+    PSet P;
+    std::string e;
+    if (n > 64 || !pset_from_flat(18, flat, len, 0, P, e)) return -1;
+    const int S = 64, nseg = (nsteps + K - 1) / K;
+    std::vector<double> st((size_t)75 * S, 0.0), ov((size_t)kOverrides * S, 1.0);
+    std::vector<int> user(S, -1);
+    for (int v = 0; v < n; ++v) {
+        user[v] = v;
+        for (int f = 0; f < 75; ++f) st[(size_t)f * S + v] = init[(size_t)v * 75 + f];
+        for (int f = 0; f < kOverrides; ++f) ov[(size_t)f * S + v] = ovr[(size_t)f * n + v];
+    }
+    std::vector<double> ckpt((size_t)nseg * kAdjCkptRow * S), tape((size_t)group * K * kAdjTapeRow * S),
+        carry((size_t)kAdjCarry * S);
+    AdjLaunch L{};
+    L.slot_user = user.data();
+    L.state = st.data();
+    L.ovr = ov.data();
+    L.ctrl = ctrl;
+    L.xy = xy;
+    L.xy_bar = xy_bar;
+    L.ctrl_bar = ctrl_bar;
+    L.state_bar = state_bar;
+    L.param_bar = param_bar;
+    L.ckpt = ckpt.data();
+    L.tape = tape.data();
+    L.carry = carry.data();
+    L.dt = 1e-3;
+    L.nsteps = nsteps;
+    L.K = K;
+    L.S = S;
+    L.n_user = n;
+    L.fwd_tape_lo = nseg - group;
+    if (lanes == 4) adjoint_group<4>(P, L, nseg, group);
+    else if (lanes == 2) adjoint_group<2>(P, L, nseg, group);
+    else adjoint_lanes(P, L, nseg, group);
+    return 0;
+}
 
 // n vehicles, nsteps >= 1 steps on `lanes` lanes per vehicle (1, 2 or 4): final records into fin[n][rec].
 // walks receives whether the group's map walk serves this parameter set.

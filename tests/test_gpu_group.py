@@ -50,3 +50,40 @@ def test_lane_groups_give_the_one_lane_bits(dof, nr, n):
     s.close()
     assert n < 64 or not np.array_equal(ref, init)
     np.testing.assert_array_equal(got, ref)
+
+
+@pytest.mark.parametrize("budget", [0, 1])
+def test_adjoint_lane_groups_give_the_one_lane_bits(budget):
+    """Trajectories and gradients of fleets at the sizes where the forward's and the reverse's lanes change,
+    against the same vehicles at the head of a fleet of more than one wavefront per SIMD (one lane each);
+    budget 1 makes every backward group a single segment, recomputed but for the last."""
+    import torch
+
+    from lfdm_amd.mpc import moving_start
+    from lfdm_amd.torch_ops import make_solver, rollout
+
+    flat = lfdm_amd.params_from_json(18, W.HMMWV_VEH, W.HMMWV_TIRE)
+    steps, big = 40, 65_600
+    g = torch.Generator(device="cuda").manual_seed(9)
+    rand = lambda *s: torch.rand(s, generator=g, dtype=torch.float64, device="cuda")  # noqa: E731
+    ctrl = torch.stack([rand(steps, big) - 0.5, rand(steps, big), 0.3 * rand(steps, big)], 1)
+    par = torch.from_numpy(W.default_overrides(flat, big)).cuda() * (0.9 + 0.2 * rand(7, big))
+    init = (moving_start(flat, 1)[0].cuda()[None] * (0.5 + rand(big, 1))).contiguous()
+    gxy = rand(steps, 2, big) - 0.5
+
+    def gradients(n):
+        s = make_solver(flat, n)
+        s.adjoint_set_tape_budget(budget)
+        x = [t[..., :n].contiguous().requires_grad_(True) for t in (ctrl, par)] + [
+            init[:n].contiguous().requires_grad_(True)]
+        xy = rollout(s, *x, 16)
+        out = [xy.detach(), *torch.autograd.grad(xy, x, gxy[..., :n].contiguous())]
+        torch.cuda.synchronize()
+        s.close()
+        return out
+
+    ref = gradients(big)
+    for n in (1, 65, 16384, 16385, 32768, 32769, 65536):
+        for name, a, b in zip(("xy", "controls", "parameters", "records"), gradients(n), ref):
+            b = b[:n] if name == "records" else b[..., :n]
+            assert torch.equal(a, b), (name, n)

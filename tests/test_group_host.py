@@ -136,3 +136,42 @@ def test_group_step_on_other_powertrains(dof, form):
         flat = with_map(flat, dof, 2, torque)
         walks = False
     check(dof, False, flat, 5 + dof, walks)
+
+
+@pytest.mark.parametrize("veh,tire,nr,walks", [v for v in VEHICLES if not v[2] and v[3]],
+                         ids=[v[0] for v in VEHICLES if not v[2] and v[3]])
+@pytest.mark.parametrize("K,group", [(60, 1), (16, 2), (7, 9)])
+def test_group_adjoint_gives_the_one_lane_bits(veh, tire, nr, walks, K, group):
+    """Forward trajectory and every gradient, with the whole tape, with recomputed groups of segments, and
+    with a ragged last segment."""
+    check_adjoint(params(18, veh, tire, nr), K, group)
+
+
+def test_group_adjoint_scans_maps_that_do_not_ascend():
+    flat = params(18, "HMMWV/vehicle.json", "HMMWV/tmeasy.json", False)
+    torque = map_of(flat, 18, 2)
+    torque[[3, 6]] = torque[[6, 3]]
+    check_adjoint(with_map(flat, 18, 2, torque), 16, 2)
+
+
+def check_adjoint(flat, K, group, steps=60):
+    recs, ovr, ctrl = inputs(18, False, flat, 77)
+    ctrl = np.ascontiguousarray(ctrl[:steps])
+    rng = np.random.Generator(np.random.PCG64(5))
+    xy_bar = rng.normal(size=(steps, 2, N))
+    L = ctypes.CDLL(LIB)
+    i, p = ctypes.c_int, ctypes.c_void_p
+    L.group_adjoint_run.argtypes = [i, p, i, p, p, i, i, i, i, p, p, p, p, p, p]
+    flat = np.ascontiguousarray(flat)
+
+    def gradients(lanes):
+        out = [np.zeros((steps, 2, N)), np.zeros((steps, 3, N)), np.zeros((75, N)), np.zeros((7, N))]
+        assert L.group_adjoint_run(lanes, flat.ctypes.data, flat.size, ovr.ctypes.data, recs.ctypes.data, N, steps, K,
+                                   group, ctrl.ctypes.data, xy_bar.ctypes.data, *[a.ctypes.data for a in out]) == 0
+        return out
+
+    ref = gradients(1)
+    assert all(np.abs(a).max() > 0 and np.isfinite(a).all() for a in ref)
+    for lanes in (2, 4):
+        for name, a, b in zip(("xy", "controls", "record", "parameters"), gradients(lanes), ref):
+            np.testing.assert_array_equal(a, b, err_msg=f"{name}, {lanes} lanes")
