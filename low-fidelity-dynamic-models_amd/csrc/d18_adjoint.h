@@ -655,9 +655,15 @@ LFDM_HD void body18_adj(const PSet& P, const Derived& u, const K18& k, const S& 
 // constants' bars accumulated into kb.
 // `to` (optional) holds the step's tire outputs from a forward pass (step18<..., CAPTURE>); without
 // it the tires' forward is recomputed here.
+// `parts` says through which parts of the step sb can reach the state: a part left out gets no bars.
+struct Parts18 {
+    int tires = 15;  // bit i: tire i
+    bool chassis = true, powertrain = true;
+};
+
 LFDM_HD void step18_adj(const PSet& P, const Derived& u, const K18& k, const S18& s0, double steering,
                         double throttle, double braking, double dt, S18b& sb, double& steerb, double& thrb,
-                        double& brkb, K18b& kb, const TireOut18* to = nullptr) {
+                        double& brkb, K18b& kb, const TireOut18* to = nullptr, const Parts18 parts = Parts18()) {
     const TireP& t = P.tire;
     // ================= forward recompute =================
     const double lat = s0.vdot + s0.wz * s0.u;
@@ -706,6 +712,9 @@ LFDM_HD void step18_adj(const PSet& P, const Derived& u, const K18& k, const S18
             rStat[i] = to->rStat[i];
             xedot[i] = to->xedot[i];
             yedot[i] = to->yedot[i];
+        } else if (!(parts.tires >> i & 1)) {
+            if (fz[i] <= 0) om[i] = 0;
+            fx[i] = fy[i] = My[i] = rStat[i] = 0;
         } else {
             double xt;
             tire_tmeasy(t, u, k, 0.0, i < 2 ? fdiv(sd, cd) : u.tan_delta_rear, fz[i], vsx[i], vsy[i], xe[i], ye[i],
@@ -759,8 +768,8 @@ LFDM_HD void step18_adj(const PSet& P, const Derived& u, const K18& k, const S18
         yedotb[i] = o.ye[i] * dt + o.yedot[i];
         omb[i] = o.omega[i];
     }
-    double gfxb[4], gfyb[4];
-    chassis18_adj(P, u, k, s0, gfx, gfy, sp, cp, dt, o, sb, kb, gfxb, gfyb);
+    double gfxb[4] = {0, 0, 0, 0}, gfyb[4] = {0, 0, 0, 0};
+    if (parts.chassis) chassis18_adj(P, u, k, s0, gfx, gfy, sp, cp, dt, o, sb, kb, gfxb, gfyb);
     // ---- tireToVehTransform (front tires rotated by delta) ----
     double fxb[4], fyb[4];
     double sdb = 0, cdb = 0;
@@ -777,7 +786,8 @@ LFDM_HD void step18_adj(const PSet& P, const Derived& u, const K18& k, const S18
         cdb += gfxb[i] * fx[i] + gfyb[i] * fy[i];
     }
     // ---- powertrain ----
-    powertrain4_adj(P, u, k.tqs, k.maxBrake, throttle, braking, s0.u, s0.crank, s0.gear, om, fx, rStat, My, pb);
+    if (parts.powertrain)
+        powertrain4_adj(P, u, k.tqs, k.maxBrake, throttle, braking, s0.u, s0.crank, s0.gear, om, fx, rStat, My, pb);
     thrb += pb.throttle;
     brkb += pb.braking;
     kb.tqs += pb.tqs;
@@ -796,6 +806,10 @@ LFDM_HD void step18_adj(const PSet& P, const Derived& u, const K18& k, const S18
             // reset: xe, ye, omega become 0 (their incoming bars stop here); xedot, yedot pass through
             sb.xedot[i] += xedotb[i];
             sb.yedot[i] += yedotb[i];
+            continue;
+        }
+        if (!(parts.tires >> i & 1)) {
+            sb.omega[i] += omb[i];
             continue;
         }
         TireBars tb;

@@ -6,7 +6,7 @@
 //    the wavefronts of the fleet and the recompute runs at full occupancy even for fleets that fill
 //    only one wavefront per SIMD.  The tape is blocked by wavefront (one contiguous 19 KB run per
 //    wavefront and step) and the per-vehicle constants sit in LDS.
-//  - step_jacobian: one lane per slot; the step's Jacobian at the current record, one step adjoint
+//  - step_jacobian: one lane per (row, slot); the step's Jacobian at the current record, one step adjoint
 //    sweep per row.
 //  - adj_reverse: one lane per slot; walks the group's segments backwards through the step adjoint
 //    of d18_adjoint.h.  The step adjoint needs the whole register file of a SIMD, so the per-vehicle
@@ -64,18 +64,20 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(1, 1))
     adj_reverse_lane(L, slot, pset_at(L.sets, uniform(L.wave_set[wave])), ks[threadIdx.x], kbs[threadIdx.x]);
 }
 
-__global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(1, 1))) void step_jacobian(AdjLaunch L) {
-    const int slot = blockIdx.x * blockDim.x + threadIdx.x;
-    const int wave = uniform(slot >> 6);
-    if (wave * kWave >= L.S) return;
-    jac_lane(L, slot, pset_at(L.sets, uniform(L.wave_set[wave])));
+// One wavefront per (row, 64 slots), the rows with most work first, each row through the parts of the step it
+// reaches.  With a vehicle's 21 rows on one lane the kernel took the latency of 21 sweeps at any size and ran a
+// fleet of 1,563 wavefronts in two rounds: 64 vehicles 580 -> 27 us, 100,003 vehicles 2,479 -> 410 us (0.98 TB/s
+// of Jacobian).  One wave per SIMD (330 VGPRs): two, with 102 spilled, measure the same.
+__global__ __launch_bounds__(kWave) __attribute__((amdgpu_waves_per_eu(1, 1))) void step_jacobian(AdjLaunch L) {
+    const int slot = blockIdx.x * kWave + threadIdx.x;
+    jac_row(L, kJacRows - 1 - (int)blockIdx.y, slot, pset_at(L.sets, uniform(L.wave_set[blockIdx.x])));
 }
 
 }  // namespace
 
 hipError_t launch_step_jacobian(const AdjLaunch& L, hipStream_t stream) {
     if (L.S <= 0) return hipSuccess;
-    hipLaunchKernelGGL(step_jacobian, (L.S + kThreads - 1) / kThreads, kThreads, 0, stream, L);
+    hipLaunchKernelGGL(step_jacobian, dim3(L.S / kWave, kJacRows), kWave, 0, stream, L);
     return hipGetLastError();
 }
 

@@ -310,7 +310,11 @@ LFDM_HD void adj_reverse_lane(const AdjLaunch& L, int slot, const PSet& P, K18& 
 // (dof18_halfImplicit.cpp:320-341); without a converter crankOmega is no state of the step (the
 // reference leaves it out): its column is zero and its row the derivative of the slaved crank speed.
 // The lagged accelerations, deflection rates and gear of the record are held at their values.
-LFDM_HD void jac_lane(const AdjLaunch& L, int slot, const PSet& P) {
+//
+// Row r of one slot.  A tire deflection's row reaches the state through its tire alone, a wheel speed's
+// through its tire and the powertrain, the crank's through the powertrain, the chassis rows through the chassis
+// and the four tires: 44 tire sweeps over the 21 rows, where sweeping every tire for every row takes 84.
+LFDM_HD void jac_row(const AdjLaunch& L, int r, int slot, const PSet& P) {
     const int user = L.slot_user[slot];
     if (user < 0) return;
     const size_t S = (size_t)L.S, N = (size_t)L.n_user;
@@ -319,36 +323,38 @@ LFDM_HD void jac_lane(const AdjLaunch& L, int slot, const PSet& P) {
     K18 k;
     load_k(P, L.ovr + slot, S, k);
     const double steer = L.ctrl[user], thr = L.ctrl[N + user], brk = L.ctrl[2 * N + user];
-    for (int r = 0; r < kJacRows; ++r) {
-        S18b sb;
-        s18b_zero(sb);
+    S18b sb;
+    s18b_zero(sb);
 #pragma unroll
-        for (int i = 0; i < 4; ++i) {
-            sb.xe[i] = r == 2 * i ? 1.0 : 0.0;
-            sb.ye[i] = r == 2 * i + 1 ? 1.0 : 0.0;
-            sb.omega[i] = r == 8 + i ? 1.0 : 0.0;
-        }
-        sb.crank = r == 12 ? 1.0 : 0.0;
-        sb.x = r == 13 ? 1.0 : 0.0;
-        sb.y = r == 14 ? 1.0 : 0.0;
-        sb.u = r == 15 ? 1.0 : 0.0;
-        sb.v = r == 16 ? 1.0 : 0.0;
-        sb.psi = r == 17 ? 1.0 : 0.0;
-        sb.wz = r == 18 ? 1.0 : 0.0;
-        sb.phi = r == 19 ? 1.0 : 0.0;
-        sb.wx = r == 20 ? 1.0 : 0.0;
-        K18b kb;
-        k18b_zero(kb);
-        double gs = 0, gt = 0, gb = 0;
-        step18_adj(P, P.d, k, s, steer, thr, brk, L.dt, sb, gs, gt, gb, kb);
-        const double col[kJacCols] = {sb.xe[0], sb.ye[0], sb.xe[1], sb.ye[1], sb.xe[2], sb.ye[2], sb.xe[3], sb.ye[3],
-                                      sb.omega[0], sb.omega[1], sb.omega[2], sb.omega[3],
-                                      P.tcbool ? sb.crank : 0.0, sb.x, sb.y, sb.u, sb.v, sb.psi, sb.wz, sb.phi, sb.wx,
-                                      gs, gt, gb};
-        double* row = L.jac + (size_t)r * kJacCols * N + user;
-#pragma unroll
-        for (int j = 0; j < kJacCols; ++j) row[(size_t)j * N] = col[j];
+    for (int i = 0; i < 4; ++i) {
+        sb.xe[i] = r == 2 * i ? 1.0 : 0.0;
+        sb.ye[i] = r == 2 * i + 1 ? 1.0 : 0.0;
+        sb.omega[i] = r == 8 + i ? 1.0 : 0.0;
     }
+    sb.crank = r == 12 ? 1.0 : 0.0;
+    sb.x = r == 13 ? 1.0 : 0.0;
+    sb.y = r == 14 ? 1.0 : 0.0;
+    sb.u = r == 15 ? 1.0 : 0.0;
+    sb.v = r == 16 ? 1.0 : 0.0;
+    sb.psi = r == 17 ? 1.0 : 0.0;
+    sb.wz = r == 18 ? 1.0 : 0.0;
+    sb.phi = r == 19 ? 1.0 : 0.0;
+    sb.wx = r == 20 ? 1.0 : 0.0;
+    Parts18 parts;
+    parts.tires = r < 8 ? 1 << (r / 2) : r < 12 ? 1 << (r - 8) : r == 12 ? 0 : 15;
+    parts.chassis = r >= 13;
+    parts.powertrain = r >= 8 && r < 13;
+    K18b kb;
+    k18b_zero(kb);
+    double gs = 0, gt = 0, gb = 0;
+    step18_adj(P, P.d, k, s, steer, thr, brk, L.dt, sb, gs, gt, gb, kb, nullptr, parts);
+    const double col[kJacCols] = {sb.xe[0], sb.ye[0], sb.xe[1], sb.ye[1], sb.xe[2], sb.ye[2], sb.xe[3], sb.ye[3],
+                                  sb.omega[0], sb.omega[1], sb.omega[2], sb.omega[3],
+                                  P.tcbool ? sb.crank : 0.0, sb.x, sb.y, sb.u, sb.v, sb.psi, sb.wz, sb.phi, sb.wx,
+                                  gs, gt, gb};
+    double* row = L.jac + (size_t)r * kJacCols * N + user;
+#pragma unroll
+    for (int j = 0; j < kJacCols; ++j) row[(size_t)j * N] = col[j];
 }
 
 }  // namespace dev

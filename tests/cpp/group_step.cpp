@@ -234,6 +234,57 @@ extern "C" int group_adjoint_run(int lanes, const double* flat, int len, const d
     return 0;
 }
 
+// Step Jacobians jac[21][24][n] of n <= 64 vehicles at their records under ctrl[3][n]: by the kernel's rows, each
+// through the parts of the step it reaches (full 0), or every row through the whole step (full 1).
+extern "C" int group_jacobian_run(int full, const double* flat, int len, const double* ovr, const double* init, int n,
+                                  const double* ctrl, double* jac) {
+    PSet P;
+    std::string e;
+    if (n > 64 || !pset_from_flat(18, flat, len, 0, P, e)) return -1;
+    const int S = 64;
+    std::vector<double> st((size_t)75 * S, 0.0), ov((size_t)kOverrides * S, 1.0);
+    std::vector<int> user(S, -1);
+    for (int v = 0; v < n; ++v) {
+        user[v] = v;
+        for (int f = 0; f < 75; ++f) st[(size_t)f * S + v] = init[(size_t)v * 75 + f];
+        for (int f = 0; f < kOverrides; ++f) ov[(size_t)f * S + v] = ovr[(size_t)f * n + v];
+    }
+    AdjLaunch L{};
+    L.slot_user = user.data();
+    L.state = st.data();
+    L.ovr = ov.data();
+    L.ctrl = ctrl;
+    L.jac = jac;
+    L.dt = 1e-3;
+    L.S = S;
+    L.n_user = n;
+    for (int v = 0; v < n; ++v)
+        for (int r = 0; r < kJacRows; ++r) {
+            if (!full) {
+                jac_row(L, r, v, P);
+                continue;
+            }
+            S18 s;
+            K18 k;
+            load_record(L.state, S, v, s);
+            load_k(P, L.ovr + v, S, k);
+            S18b b;
+            K18b kb;
+            s18b_zero(b);
+            k18b_zero(kb);
+            double* seed[kJacRows] = {&b.xe[0], &b.ye[0], &b.xe[1], &b.ye[1], &b.xe[2], &b.ye[2], &b.xe[3],
+                                      &b.ye[3], &b.omega[0], &b.omega[1], &b.omega[2], &b.omega[3], &b.crank, &b.x,
+                                      &b.y, &b.u, &b.v, &b.psi, &b.wz, &b.phi, &b.wx};
+            *seed[r] = 1.0;
+            double g[3] = {0, 0, 0};
+            step18_adj(P, P.d, k, s, ctrl[v], ctrl[n + v], ctrl[2 * n + v], L.dt, b, g[0], g[1], g[2], kb);
+            double* row = jac + (size_t)r * kJacCols * n + v;
+            for (int c = 0; c < kJacRows; ++c) row[(size_t)c * n] = c == 12 && !P.tcbool ? 0.0 : *seed[c];
+            for (int c = 0; c < 3; ++c) row[(size_t)(kJacRows + c) * n] = g[c];
+        }
+    return 0;
+}
+
 // n vehicles, nsteps >= 1 steps on `lanes` lanes per vehicle (1, 2 or 4): final records into fin[n][rec].
 // walks receives whether the group's map walk serves this parameter set.
 extern "C" int group_step_run(int dof, int nr, int lanes, const double* flat, int len, const double* ovr,

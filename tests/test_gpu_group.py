@@ -87,3 +87,34 @@ def test_adjoint_lane_groups_give_the_one_lane_bits(budget):
         for name, a, b in zip(("xy", "controls", "parameters", "records"), gradients(n), ref):
             b = b[:n] if name == "records" else b[..., :n]
             assert torch.equal(a, b), (name, n)
+
+
+def test_step_jacobian_does_not_depend_on_the_fleet():
+    """Jacobians of 1, 64 and 65 vehicles are those of the same vehicles in a fleet of 200."""
+    import torch
+
+    from lfdm_amd.mpc import moving_start
+    from lfdm_amd.torch_ops import make_solver
+
+    flat = lfdm_amd.params_from_json(18, W.HMMWV_VEH, W.HMMWV_TIRE)
+    big = 200
+    g = torch.Generator(device="cuda").manual_seed(4)
+    init = (moving_start(flat, 1)[0].cuda()[None] *
+            (0.5 + torch.rand((big, 1), generator=g, dtype=torch.float64, device="cuda"))).contiguous()
+    ctrl = torch.rand((3, big), generator=g, dtype=torch.float64, device="cuda")
+
+    def jacobian(n):
+        s = make_solver(flat, n)
+        s.set_states_device(init[:n].contiguous().data_ptr())
+        c = ctrl[:, :n].contiguous()
+        jac = torch.full((21, 24, n), float("nan"), dtype=torch.float64, device="cuda")
+        torch.cuda.synchronize()
+        assert s.step_jacobian(c.data_ptr(), jac.data_ptr()) == (21, 24)
+        s.synchronize()
+        s.close()
+        return jac
+
+    ref = jacobian(big)
+    assert torch.isfinite(ref).all()
+    for n in (1, 64, 65):
+        assert torch.equal(jacobian(n), ref[..., :n]), n

@@ -175,3 +175,26 @@ def check_adjoint(flat, K, group, steps=60):
     for lanes in (2, 4):
         for name, a, b in zip(("xy", "controls", "record", "parameters"), gradients(lanes), ref):
             np.testing.assert_array_equal(a, b, err_msg=f"{name}, {lanes} lanes")
+
+
+@pytest.mark.parametrize("veh,tire,nr,walks", [v for v in VEHICLES if not v[2] and v[3]],
+                         ids=[v[0] for v in VEHICLES if not v[2] and v[3]])
+def test_jacobian_rows_equal_the_whole_steps(veh, tire, nr, walks):
+    """A row swept only through the parts of the step it reaches has the values of the sweep through all of
+    them, at rest, moving, braking and with wheels off the ground."""
+    flat = np.ascontiguousarray(params(18, veh, tire, nr))
+    recs, ovr, ctrl = inputs(18, False, flat, 31)
+    recs, _ = run(18, False, 1, flat, recs, ovr, ctrl)
+    recs[0] = 0.0
+    lagged = [i for i, f in enumerate(lfdm_amd.record_fields(18)) if f == "vdot"][0]
+    recs[1, lagged] = 60.0  # a lateral acceleration that lifts the left wheels
+    ctl = np.ascontiguousarray(ctrl[-1])
+    L = ctypes.CDLL(LIB)
+    i, p = ctypes.c_int, ctypes.c_void_p
+    L.group_jacobian_run.argtypes = [i, p, i, p, p, i, p, p]
+    J = [np.zeros((21, 24, N)) for _ in range(2)]
+    for full in (0, 1):
+        assert L.group_jacobian_run(full, flat.ctypes.data, flat.size, ovr.ctypes.data, recs.ctypes.data, N,
+                                    ctl.ctypes.data, J[full].ctypes.data) == 0
+    assert np.isfinite(J[1]).all()
+    np.testing.assert_array_equal(J[0], J[1])
