@@ -1,0 +1,133 @@
+// A copy into pageable memory goes through the runtime's staging buffer and one thread's memcpy, which also
+// takes the page faults of memory the caller has just allocated: 10 GB/s for the 600 MB of a 1,000,000-vehicle
+// fleet's records, where the link moves 57 GB/s.  Here several threads each take a part of the array
+// through two pinned buffers of their own, so that the link, the faults and the copies of different parts
+// overlap.
+#include "copy_out.h"
+
+#include <algorithm>
+#include <atomic>
+#include <cstring>
+#include <mutex>
+#include <thread>
+#include <vector>
+
+namespace lfdm {
+
+namespace {
+
+// 16 buffers of 2 MiB: a part takes about 40 us on the link and ten times that to be copied out by one thread.
+// 600 MB (GB/s): 8 threads with parts of 1 MiB 30, of 2 MiB 35; 12 or 16 threads 29 (parts of 0.5 MiB 21).
+constexpr int kThreads = 8, kBuffers = 2;
+constexpr size_t kPart = size_t(2) << 20;
+// Below this the threads' start-up costs more than they save.
+constexpr size_t kLeast = size_t(4) << 20;
+
+std::mutex g_lock;  // guards everything here; a copy holds it, a second one at the time goes the plain way
+char* g_pinned = nullptr;  // kThreads x kBuffers parts
+char* g_small = nullptr;   // kStagedBytes
+int g_holders = 0;
+
+// One thread's share: every kThreads-th part.
+hipError_t copy_parts(int device, char* dst, const char* src, size_t n, int first, hipStream_t stream) {
+    hipError_t e = hipSetDevice(device);
+    hipEvent_t done[kBuffers] = {};
+    for (int b = 0; b < kBuffers && e == hipSuccess; ++b) e = hipEventCreateWithFlags(&done[b], hipEventDisableTiming);
+    char* const pinned = g_pinned + (size_t)first * kBuffers * kPart;
+    const size_t parts = (n + kPart - 1) / kPart;
+    const auto size = [&](size_t p) { return std::min(kPart, n - p * kPart); };
+    const auto request = [&](size_t p, int b) {
+        hipError_t r = hipMemcpyAsync(pinned + b * kPart, src + p * kPart, size(p), hipMemcpyDeviceToHost, stream);
+        return r == hipSuccess ? hipEventRecord(done[b], stream) : r;
+    };
+    int b = 0;
+    if (e == hipSuccess && (size_t)first < parts) e = request(first, b);
+    for (size_t p = first; p < parts && e == hipSuccess; p += kThreads, b = (b + 1) % kBuffers) {
+        if (p + kThreads < parts) e = request(p + kThreads, (b + 1) % kBuffers);
+        const hipError_t w = hipEventSynchronize(done[b]);
+        if (e == hipSuccess) e = w;
+        if (e == hipSuccess) std::memcpy(dst + p * kPart, pinned + b * kPart, size(p));
+    }
+    // no request may still be writing the buffers when they go back
+    if (e != hipSuccess) (void)hipStreamSynchronize(stream);
+    for (hipEvent_t d : done)
+        if (d) (void)hipEventDestroy(d);
+    return e;
+}
+
+bool ensure(char*& p, size_t n) {
+    if (!p && hipHostMalloc((void**)&p, n, hipHostMallocPortable) != hipSuccess) {
+        p = nullptr;
+        (void)hipGetLastError();  // the plain way is taken instead
+    }
+    return p != nullptr;
+}
+
+// Whether the runtime knows nothing of dst: neither pinned (which the link reaches without staging) nor
+// device memory.
+bool ordinary(const void* dst) {
+    hipPointerAttribute_t a{};
+    if (hipPointerGetAttributes(&a, dst) == hipSuccess) return a.type == hipMemoryTypeUnregistered;
+    (void)hipGetLastError();
+    return true;
+}
+
+hipError_t plain(void* dst, const void* src, size_t n, hipStream_t stream) {
+    const hipError_t e = hipMemcpyAsync(dst, src, n, hipMemcpyDeviceToHost, stream);
+    return e == hipSuccess ? hipStreamSynchronize(stream) : e;
+}
+
+}  // namespace
+
+char* copy_out_begin(const void* dst, size_t n) {
+    if (n > kStagedBytes || !ordinary(dst) || !g_lock.try_lock()) return nullptr;
+    if (!ensure(g_small, kStagedBytes)) {
+        g_lock.unlock();
+        return nullptr;
+    }
+    return g_small;
+}
+
+void copy_out_end() { g_lock.unlock(); }
+
+hipError_t copy_out(void* dst, const void* device_src, size_t n, hipStream_t stream) {
+    std::unique_lock<std::mutex> lock(g_lock, std::defer_lock);
+    int device = 0;
+    if (n < kLeast || !ordinary(dst) || hipGetDevice(&device) != hipSuccess || !lock.try_lock() ||
+        !ensure(g_pinned, kThreads * kBuffers * kPart))
+        return plain(dst, device_src, n, stream);
+    hipError_t result[kThreads];
+    std::vector<std::thread> helpers;
+    int started = 1;  // this thread takes the first share
+    try {
+        helpers.reserve(kThreads);
+        for (; started < kThreads; ++started)
+            helpers.emplace_back([&, k = started] {
+                result[k] = copy_parts(device, (char*)dst, (const char*)device_src, n, k, stream);
+            });
+    } catch (...) {  // no more threads: the shares left over are this thread's too
+    }
+    result[0] = copy_parts(device, (char*)dst, (const char*)device_src, n, 0, stream);
+    for (int k = started; k < kThreads; ++k)
+        result[k] = copy_parts(device, (char*)dst, (const char*)device_src, n, k, stream);
+    for (std::thread& t : helpers) t.join();
+    for (hipError_t e : result)
+        if (e != hipSuccess) return e;
+    return hipSuccess;
+}
+
+void copy_out_hold() {
+    std::lock_guard<std::mutex> lock(g_lock);
+    ++g_holders;
+}
+
+void copy_out_release() {
+    std::lock_guard<std::mutex> lock(g_lock);
+    if (--g_holders > 0) return;
+    for (char** p : {&g_pinned, &g_small}) {
+        if (*p) (void)hipHostFree(*p);
+        *p = nullptr;
+    }
+}
+
+}  // namespace lfdm

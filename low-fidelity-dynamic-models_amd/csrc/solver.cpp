@@ -20,6 +20,7 @@
 #include <vector>
 
 #include "../../include/lfdm_amd.h"
+#include "copy_out.h"
 #include "kernels.h"
 #include "params.h"
 
@@ -672,6 +673,7 @@ int lfdm_create(int dof, unsigned total, lfdm_solver** out) {
         return fail(LFDM_E_UNSUPPORTED, "unsupported model: " + std::to_string(dof) + "-DOF");
     if (total == 0) return fail(LFDM_E_ARG, "total vehicle count must be positive");
     lfdm_solver* h = new lfdm_solver();
+    copy_out_hold();
     h->dof = dof;
     h->total = total;
     *out = h;
@@ -703,6 +705,7 @@ int lfdm_destroy(lfdm_solver* h) {
     if (h->ev0) (void)hipEventDestroy(h->ev0);
     if (h->ev1) (void)hipEventDestroy(h->ev1);
     if (h->own_stream && h->stream) (void)hipStreamDestroy(h->stream);
+    copy_out_release();
     delete h;
     return LFDM_OK;
 }
@@ -1010,11 +1013,20 @@ int lfdm_get_states(lfdm_solver* h, double* records) {
         return LFDM_OK;
     }
     const size_t need = (size_t)h->total * h->rec;
+    // a small fleet's records: gathered straight into pinned memory, without a copy of its own behind the gather
+    if (char* staged = copy_out_begin(records, need * sizeof(double))) {
+        hipError_t e = launch_gather(h->d_state, h->S, h->rec, h->d_user_slot, (int)h->total,
+                                     reinterpret_cast<double*>(staged), h->stream);
+        if (e == hipSuccess) e = hipStreamSynchronize(h->stream);
+        if (e == hipSuccess) std::memcpy(records, staged, need * sizeof(double));
+        copy_out_end();
+        if (e != hipSuccess) return fail(LFDM_E_HIP, hipGetErrorString(e));
+        return LFDM_OK;
+    }
     if (int rc = ensure_buffer(h->d_rec, h->rec_cap, need)) return rc;
     hipError_t e = launch_gather(h->d_state, h->S, h->rec, h->d_user_slot, (int)h->total, h->d_rec, h->stream);
     if (e != hipSuccess) return fail(LFDM_E_HIP, hipGetErrorString(e));
-    HIPCHK(hipMemcpyAsync(records, h->d_rec, need * sizeof(double), hipMemcpyDeviceToHost, h->stream));
-    HIPCHK(hipStreamSynchronize(h->stream));
+    HIPCHK(copy_out(records, h->d_rec, need * sizeof(double), h->stream));
     return LFDM_OK;
 }
 
