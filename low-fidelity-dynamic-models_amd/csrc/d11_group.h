@@ -48,11 +48,11 @@ LFDM_HD void move11g(S11g& s, double sp, double cp, double dt) {
 
 // step11 without its closing position update; `lag`: the previous step's position update comes first
 // (its sine and cosine of the yaw angle from lane 1 while lane 0 takes the steering angle's).
-template <bool NR, bool FULL>
-LFDM_HD void step11g(const PSet& P, const Derived& u, const K11g& k, S11g& s, double steering, double throttle,
+template <bool NR, bool FULL, class PS>
+LFDM_HD void step11g(const PS& P, const Derived& u, const K11g& k, S11g& s, double steering, double throttle,
                      double braking, double dt, bool lag, X11g* x) {
     const TireP& t = P.tire;
-    const double delta = P.nonLinearSteer ? map_y<false>(P.steer, steering) : steering * P.maxSteer;
+    const double delta = P.nonLinearSteer ? map_y<false>(full_set(P).steer, steering) : steering * P.maxSteer;
     double sa, ca;
     sincos_fast((s.q & 1) ? s.psi : delta, sa, ca);
     const double sd = group_value<2, 0>(sa), cd = group_value<2, 0>(ca);

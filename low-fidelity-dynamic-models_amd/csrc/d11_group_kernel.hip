@@ -4,8 +4,8 @@
 namespace lfdm {
 
 hipError_t launch_d11_group(const Launch& L, int block, hipStream_t stream) {
-    if (L.waves == 1) return kern::launch_tire<kern::M11g, 1>(L, block, stream);
-    return kern::launch_tire<kern::M11g, 2>(L, block, stream);
+    if (L.waves == 1) return kern::launch_tire<kern::M11g<true>, 1>(L, block, stream);
+    return kern::launch_tire<kern::M11g<false>, 2>(L, block, stream);
 }
 
 }  // namespace lfdm

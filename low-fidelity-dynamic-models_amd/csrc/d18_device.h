@@ -120,8 +120,8 @@ struct TireOut18 {
 };
 
 // computeVehRHS (dof18.cpp:1019-1078): chassis accelerations from the tire forces in the vehicle's axes.
-template <bool STRICT>
-LFDM_HD void chassis18(const PSet& P, const Derived& d, const K18& k, double u, double v, double wz, double wx,
+template <bool STRICT, class PS>
+LFDM_HD void chassis18(const PS& P, const Derived& d, const K18& k, double u, double v, double wz, double wx,
                        double phi, const double* fx, const double* fy, double& udot, double& vdot, double& wxdot,
                        double& wzdot) {
     const double E1 = k.neg_mt * wz * u + (fy[0] + fy[1] + fy[2] + fy[3]);

@@ -61,9 +61,9 @@ LFDM_HD void move18g(S18g<G>& s, double sp, double cp, double dt) {
 
 // The step's steering angle, with the previous step's position update (`lag`): one lane takes the sine and
 // cosine of the steering angle while another takes the yaw angle's.
-template <int G>
-LFDM_HD void angles18g(const PSet& P, S18g<G>& s, double steering, double dt, bool lag, double& sd, double& cd) {
-    const double delta = P.nonLinearSteer ? map_y<false>(P.steer, steering) : steering * P.maxSteer;
+template <int G, class PS>
+LFDM_HD void angles18g(const PS& P, S18g<G>& s, double steering, double dt, bool lag, double& sd, double& cd) {
+    const double delta = P.nonLinearSteer ? map_y<false>(full_set(P).steer, steering) : steering * P.maxSteer;
     double sa, ca;
     sincos_fast((s.q & 1) ? s.psi : delta, sa, ca);
     sd = group_value<G, 0>(sa);
@@ -108,8 +108,8 @@ LFDM_HD double patch18g(const K18g<G>& k, double u, double v, double wz, double 
 }
 
 // step18 without its closing position update, after angles18g.
-template <bool NR, bool FULL, int G, bool CAPTURE = false>
-LFDM_HD void step18g(const PSet& P, const Derived& u, const K18& c, const K18g<G>& k, S18g<G>& s, double sd, double cd,
+template <bool NR, bool FULL, int G, bool CAPTURE = false, class PS>
+LFDM_HD void step18g(const PS& P, const Derived& u, const K18& c, const K18g<G>& k, S18g<G>& s, double sd, double cd,
                      double throttle, double braking, double dt, X18g<G>* x, TireOut18g<G>* to = nullptr) {
     constexpr int N = 4 / G;
     const TireP& t = P.tire;

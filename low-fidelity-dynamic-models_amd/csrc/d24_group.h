@@ -71,13 +71,13 @@ LFDM_HD void move24g(S24g<G>& s, double sp, double cp, double dt) {
 // step24 without its closing position update; `lag`: the previous step's position update comes first.
 // The four angles' sines and cosines (pitch, roll, steering and, for the lagging update, yaw) are shared
 // out: one angle per lane of four, two per lane of two.
-template <bool NR, bool FULL, int G>
-LFDM_HD void step24g(const PSet& P, const Derived& u, const K24g<G>& k, S24g<G>& s, double steering, double throttle,
+template <bool NR, bool FULL, int G, class PS>
+LFDM_HD void step24g(const PS& P, const Derived& u, const K24g<G>& k, S24g<G>& s, double steering, double throttle,
                      double braking, double dt, bool lag, X24g<G>* x) {
     constexpr int N = 4 / G;
     const TireP& t = P.tire;
     const double a = P.a, b = P.b;
-    const double delta = P.nonLinearSteer ? map_y<false>(P.steer, steering) : steering * P.maxSteer;
+    const double delta = P.nonLinearSteer ? map_y<false>(full_set(P).steer, steering) : steering * P.maxSteer;
     double sth, cth, sph, cph, sd, cd;
     if constexpr (G == 4) {
         double sa, ca;

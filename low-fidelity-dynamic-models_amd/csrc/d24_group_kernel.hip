@@ -5,10 +5,10 @@ namespace lfdm {
 
 hipError_t launch_d24_group(const Launch& L, int block, hipStream_t stream) {
     if (L.lanes == 4) {
-        if (L.waves == 1) return kern::launch_tire<kern::M24g<4>, 1>(L, block, stream);
-        return kern::launch_tire<kern::M24g<4>, 2>(L, block, stream);
+        if (L.waves == 1) return kern::launch_tire<kern::M24g<4, true>, 1>(L, block, stream);
+        return kern::launch_tire<kern::M24g<4, false>, 2>(L, block, stream);
     }
-    return kern::launch_tire<kern::M24g<2>, 2>(L, block, stream);
+    return kern::launch_tire<kern::M24g<2, false>, 2>(L, block, stream);
 }
 
 }  // namespace lfdm

@@ -416,25 +416,53 @@ LFDM_HD double map_y_scaled(const Map& m, double x, double sx, double sy1, doubl
     return x <= F.x * sx ? F.y * sy1 * sy2 : (x >= B.x * sx ? B.y * sy1 * sy2 : y);
 }
 
-// Driver-table lookup at a wave-uniform time (utils.cpp:34-56).
-LFDM_HD void driver_input(double t, const DrvRow* __restrict__ rows, int n, double& s, double& th,
-                                             double& b) {
-    if (t <= rows[0].t) {
-        s = rows[0].steering; th = rows[0].throttle; b = rows[0].braking;
-        return;
+// Where the last lookup in a driver table ended: its row, and, with AHEAD, the rows around it and the table's
+// ends, held so that the next lookup loads nothing until the time passes the row.
+template <bool AHEAD>
+struct DrvWalk {
+    int r = -1;  // none yet
+    DrvRow lo, hi, last;
+    double first;
+};
+
+// Driver-table lookup (utils.cpp:34-56) at a wave-uniform time.  The row is walked to from the last lookup's
+// instead of scanned for from the table's start, whose loads wait for each other: where the times ascend, every
+// row before it stays behind the time, whatever the table's order.  Other times scan.
+template <bool AHEAD>
+LFDM_HD void driver_input(double t, const DrvRow* __restrict__ rows, int n, bool ascending, DrvWalk<AHEAD>& w,
+                          double& s, double& th, double& b) {
+    const bool scan = w.r < 0 || !ascending;
+    int r = scan ? 1 : w.r;
+    DrvRow lo, hi, last;
+    double first;
+    if (AHEAD && !scan) {
+        lo = w.lo; hi = w.hi; last = w.last; first = w.first;
+    } else {
+        first = rows[0].t;
+        last = rows[n - 1];
+        lo = rows[r - 1];
+        hi = rows[n > 1 ? r : 0];
     }
-    if (t >= rows[n - 1].t) {
-        s = rows[n - 1].steering; th = rows[n - 1].throttle; b = rows[n - 1].braking;
-        return;
+    if (t <= first) {
+        const DrvRow f = rows[0];
+        s = f.steering; th = f.throttle; b = f.braking;
+    } else if (t >= last.t) {
+        s = last.steering; th = last.throttle; b = last.braking;
+    } else {
+        while (r < n - 1 && hi.t < t) {
+            ++r;
+            lo = hi;
+            hi = rows[r];
+        }
+        const double tbar = qdiv(t - lo.t, hi.t - lo.t);
+        s = lo.steering + tbar * (hi.steering - lo.steering);
+        th = lo.throttle + tbar * (hi.throttle - lo.throttle);
+        b = lo.braking + tbar * (hi.braking - lo.braking);
     }
-    int r = 1;
-    while (r < n - 1 && rows[r].t < t) ++r;
-    const DrvRow L = rows[r - 1];
-    const DrvRow R = rows[r];
-    const double tbar = qdiv(t - L.t, R.t - L.t);
-    s = L.steering + tbar * (R.steering - L.steering);
-    th = L.throttle + tbar * (R.throttle - L.throttle);
-    b = L.braking + tbar * (R.braking - L.braking);
+    w.r = r;
+    if (AHEAD) {
+        w.lo = lo; w.hi = hi; w.last = last; w.first = first;
+    }
 }
 
 // Gear-indexed reads by a per-lane gear over a wave-uniform table (select chain, no memory).

@@ -457,7 +457,8 @@ LFDM_HD void powertrain_torque(const PSet& P, const Derived& u, double tqs, doub
 }
 
 // The shaft torque's share of the front and the rear axle.
-LFDM_HD void axle_torques(const PSet& P, double torque_t, double& tf, double& trr) {
+template <class PS>
+LFDM_HD void axle_torques(const PS& P, double torque_t, double& tf, double& trr) {
     if (P.driveType) {
         tf = torque_t * 0.5;
         trr = torque_t * 0.5;

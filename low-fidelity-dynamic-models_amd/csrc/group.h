@@ -137,13 +137,64 @@ LFDM_HD bool group_walks(const PSet& P) {
     return !P.throttleMod && P.torque.sorted && P.losses.sorted && P.cfmap.sorted && P.trmap.sorted;
 }
 
+// The parameters a group step reads every step, held in the lane's registers.  A lone wavefront that fetches
+// them through the scalar cache step by step waits for it some 28 times a step, a quarter of its time, and may
+// use 512 registers: per step 2.69 -> 2.54 us (18-DOF, 16,384 vehicles, knots), 3.41 -> 3.24 (24-DOF), 2.62 ->
+// 2.42 (11-DOF, 32,768).  Kernels of two wavefronts per SIMD, which hide each other's waits, have no room for
+// them.  `full` has the maps and gears.
+struct HotSet {
+    double a, b, cf, cr, jxz, hrcf, hrcr, ks, bs, maxSteer;
+    int nonLinearSteer, tcbool, driveType, whichWheels, ngears;
+    TireP tire;
+    Derived d;
+    const PSet* full;
+};
+
+// Makes every double of t a register's value that the compiler cannot fetch again.
+template <class T>
+LFDM_HD void hold(T& t) {
+    static_assert(sizeof(T) % sizeof(double) == 0, "doubles only");
+    double* p = reinterpret_cast<double*>(&t);
+#pragma unroll
+    for (int i = 0; i < (int)(sizeof(T) / sizeof(double)); ++i) opaque(p[i]);
+}
+
+LFDM_HD void hot_init(const PSet& P, HotSet& h) {
+    h.a = P.a; h.b = P.b; h.cf = P.cf; h.cr = P.cr; h.jxz = P.jxz; h.hrcf = P.hrcf; h.hrcr = P.hrcr;
+    h.ks = P.ks; h.bs = P.bs; h.maxSteer = P.maxSteer;
+    h.nonLinearSteer = P.nonLinearSteer; h.tcbool = P.tcbool; h.driveType = P.driveType;
+    h.whichWheels = P.whichWheels; h.ngears = P.ngears;
+    h.tire = P.tire;
+    h.d = P.d;
+    h.full = &P;
+    for (double* v : {&h.a, &h.b, &h.cf, &h.cr, &h.jxz, &h.hrcf, &h.hrcr, &h.ks, &h.bs, &h.maxSteer}) opaque(*v);
+    hold(h.tire);
+    hold(h.d);
+}
+
+LFDM_HD const PSet& full_set(const PSet& P) { return P; }
+LFDM_HD const PSet& full_set(const HotSet& h) { return *h.full; }
+
+// The parameters a step reads: the set itself, or its HotSet in registers.
+template <bool HOT>
+struct Params {
+    HotSet h;
+    LFDM_HD void init(const PSet& P) { hot_init(P, h); }
+    LFDM_HD const HotSet& of(const PSet&) const { return h; }
+};
+template <>
+struct Params<false> {
+    LFDM_HD void init(const PSet&) {}
+    LFDM_HD const PSet& of(const PSet& P) const { return P; }
+};
+
 // powertrain_torque with the lookups and the gear's values of this vehicle's lanes.
-template <int G>
-LFDM_HD void powertrain_group(const PSet& P, const Derived& u, double tqs, double throttle, double vel_u, double mean,
+template <int G, class PS>
+LFDM_HD void powertrain_group(const PS& P, const Derived& u, double tqs, double throttle, double vel_u, double mean,
                               int q, bool walks, Walks<G>& w, GearRow& g, double& crank, int& gear,
                               double& torque_t, double& dcrank) {
     if (!walks) {
-        powertrain_torque<false>(P, u, tqs, throttle, vel_u, mean, crank, gear, torque_t, dcrank);
+        powertrain_torque<false>(full_set(P), u, tqs, throttle, vel_u, mean, crank, gear, torque_t, dcrank);
         return;
     }
     const MapXY La = w.a.e[w.a.r - 1], Ra = w.a.e[w.a.r];
@@ -197,7 +248,7 @@ LFDM_HD void powertrain_group(const PSet& P, const Derived& u, double tqs, doubl
     } else if (omega_out < g.down) {
         if (gear > 0) gear--;
     }
-    if (gear != was) gear_row(P, gear, g);
+    if (gear != was) gear_row(full_set(P), gear, g);
 }
 
 }  // namespace dev

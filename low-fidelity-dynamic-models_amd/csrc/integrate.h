@@ -32,35 +32,54 @@ struct NoControls {
     __device__ void eval(double, int, double&, double&, double&) {}
 };
 
-template <int MODE>
+// AHEAD (kernels of one wavefront per SIMD, which nothing else keeps busy while a load is under way and whose
+// lanes have registers to spare): the driver rows of the current time and the next step's per-step controls are
+// held.  With HotSet, per step: 11-DOF driver table 2.77 -> 2.16 us (16,384 vehicles), 24-DOF 3.23 -> 2.74
+// (4,096), 18-DOF per-step controls 2.75 -> 2.41 (1,024).  At two wavefronts per SIMD it cost the 24-DOF step
+// 5 % (65,536 vehicles, table: 6.65 -> 7.05).
+template <int MODE, bool AHEAD>
 struct CtrlState {
-    int kcur = -1;
+    int kcur = -1;  // the knot segment held
     double s0 = 0, s1 = 0, thr = 0, brk = 0;
+    DrvWalk<AHEAD> drv;
+    Ctl next;
+    int knext = -1;  // the step `next` is for
 };
 
-// Per-vehicle control buffers are indexed by user vehicle index `uv` with stride n_user.
-template <int MODE, class F>
-__device__ __forceinline__ Ctl controls_at(const Launch& L, const PSet& P, CtrlState<MODE>& cs, int uv, int k,
-                                           double t, F& f) {
+__device__ __forceinline__ Ctl step_controls(const Launch& L, int uv, int k) {
+    Ctl c;
+    if (L.steps_shared) {  // wave-uniform: one row per step for the whole fleet
+        const double* p = L.steps + (size_t)k * 3;
+        c.s = p[0];
+        c.th = p[1];
+        c.b = p[2];
+    } else {
+        const size_t N = (size_t)L.n_user;
+        const double* p = L.steps + (size_t)k * 3 * N + uv;
+        c.s = p[0];
+        c.th = p[N];
+        c.b = p[2 * N];
+    }
+    return c;
+}
+
+// Controls of step k at time t.  Per-vehicle control buffers are indexed by user vehicle index `uv` with stride
+// n_user; `more`: step k + 1 of this lane follows in this launch.
+template <int MODE, bool AHEAD, class F>
+__device__ __forceinline__ Ctl controls_at(const Launch& L, const PSet& P, CtrlState<MODE, AHEAD>& cs, int uv, int k,
+                                           double t, F& f, bool more = false) {
     Ctl c;
     if constexpr (MODE == kCtrlFunctor) {
         f.eval(t, uv, c.s, c.th, c.b);
     } else if (MODE == kCtrlConst) {
         c.s = L.c_s; c.th = L.c_t; c.b = L.c_b;
     } else if (MODE == kCtrlTable) {
-        driver_input(t, L.drv + P.drv_off, P.drv_rows, c.s, c.th, c.b);
+        driver_input(t, L.drv + P.drv_off, P.drv_rows, L.dt >= 0, cs.drv, c.s, c.th, c.b);
     } else if (MODE == kCtrlSteps) {
-        if (L.steps_shared) {  // wave-uniform: one row per step for the whole fleet
-            const double* p = L.steps + (size_t)k * 3;
-            c.s = p[0];
-            c.th = p[1];
-            c.b = p[2];
-        } else {
-            const size_t N = (size_t)L.n_user;
-            const double* p = L.steps + (size_t)k * 3 * N + uv;
-            c.s = p[0];
-            c.th = p[N];
-            c.b = p[2 * N];
+        c = AHEAD && cs.knext == k ? cs.next : step_controls(L, uv, k);
+        if (AHEAD && more) {
+            cs.next = step_controls(L, uv, k + 1);
+            cs.knext = k + 1;
         }
     } else {  // kCtrlKnots
         const size_t N = (size_t)L.n_user;
@@ -98,7 +117,8 @@ struct M18 {
     static constexpr int kCh = 13;
     static constexpr int kWaves = kMaxWaves18;
     static constexpr bool kKInLds = true;
-    static constexpr int kLanes = 1;  // lanes per vehicle
+    static constexpr int kLanes = 1;            // lanes per vehicle
+    static constexpr bool kAhead = false;  // CtrlState
     template <bool NR>
     struct R {
         static constexpr int kTire = NR ? 11 : 15, kVeh = 4 * kTire, om = NR ? 0 : 4;
@@ -174,7 +194,8 @@ struct M11 {
     static constexpr int kCh = 9;
     static constexpr int kWaves = kMaxWaves11;
     static constexpr bool kKInLds = true;
-    static constexpr int kLanes = 1;  // lanes per vehicle
+    static constexpr int kLanes = 1;            // lanes per vehicle
+    static constexpr bool kAhead = false;  // CtrlState
     template <bool NR>
     struct R {
         static constexpr int kTire = NR ? 11 : 15, kVeh = 2 * kTire, om = NR ? 0 : 4;
@@ -250,7 +271,8 @@ struct M24 {
     static constexpr int kCh = 15;
     static constexpr int kWaves = kMaxWaves24;
     static constexpr bool kKInLds = true;
-    static constexpr int kLanes = 1;  // lanes per vehicle
+    static constexpr int kLanes = 1;            // lanes per vehicle
+    static constexpr bool kAhead = false;  // CtrlState
     template <bool NR>
     struct R {
         static constexpr int kTire = NR ? 19 : 23, kSus = 4 * kTire, kVeh = kSus + 4 * 24, om = NR ? 0 : 4;
@@ -410,7 +432,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(W, W))) voi
     }
     const int user = L.slot_user[slot];
     const int uv = user >= 0 ? user : 0;  // padding lanes read vehicle 0's controls
-    CtrlState<MODE> cs;
+    CtrlState<MODE, M::kAhead> cs;
     double t = L.t0;  // this vehicle's time
     const double dt = L.dt;
     // output rows after fewer steps than the vehicle's last are written as the wavefront passes
@@ -429,11 +451,11 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(W, W))) voi
         if (kk < my - 1) {
             // kk != clean: the same branch on every lane
             if constexpr (M::kLanes > 1) {
-                const Ctl c = controls_at<MODE>(L, P, cs, uv, kk, t, f);
+                const Ctl c = controls_at(L, P, cs, uv, kk, t, f, true);
                 M::template step<NR, false>(P, u, k, s, c, dt, kk != clean, nullptr);
             } else {
                 if (kk != clean) M::template position<STRICT>(s, dt);
-                const Ctl c = controls_at<MODE>(L, P, cs, uv, kk, t, f);
+                const Ctl c = controls_at(L, P, cs, uv, kk, t, f);
                 M::template step<NR, false, STRICT, false>(P, u, k, s, c, dt, nullptr);
             }
             pend = true;
@@ -454,8 +476,8 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(W, W))) voi
     // whose horizon comes earlier than its wavefront's takes it at its own step and time)
     if (my > 0) {
         typename M::X x;
-        CtrlState<MODE> cl;
-        const Ctl c = controls_at<MODE>(L, P, my == wsteps ? cs : cl, uv, my - 1, t, f);
+        if (my != wsteps) cs.kcur = cs.knext = cs.drv.r = -1;  // what the wavefront's later steps left is not this lane's
+        const Ctl c = controls_at(L, P, cs, uv, my - 1, t, f);
         if constexpr (M::kLanes > 1) M::template step<NR, true>(P, u, k, s, c, dt, false, &x);
         else M::template step<NR, true, STRICT, false>(P, u, k, s, c, dt, &x);
         M::template position<STRICT>(s, dt);

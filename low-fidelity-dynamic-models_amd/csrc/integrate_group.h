@@ -10,17 +10,20 @@
 namespace lfdm {
 namespace kern {
 
-template <int G>
+// HOT: the set's parameters in registers (HotSet).
+template <int G, bool HOT>
 struct M18g {
     using S = S18g<G>;
     using X = X18g<G>;
     struct K {
         K18 c;
         K18g<G> g;
+        Params<HOT> set;
     };
     static constexpr int kCh = M18::kCh;
     static constexpr bool kKInLds = false;  // a lane's registers hold its constants
     static constexpr int kLanes = G;
+    static constexpr bool kAhead = HOT;
     static constexpr int N = S::N;
     template <bool NR>
     static LFDM_HD void load(const double* st, size_t S_, int slot, S& s, K&) {
@@ -47,15 +50,17 @@ struct M18g {
     static LFDM_HD void kinit(const PSet& P, const double* o, size_t S_, const MapXY* tab, S& s, K& k) {
         M18::kinit(P, o, S_, k.c);
         k18g_init<G>(P, k.c, s.q, k.g);
+        k.set.init(P);
         walks_init<G>(P, tab, k.c.tqs, s.q, s.maps);
         gear_row(P, s.gear, s.row);
     }
     template <bool NR, bool FULL>
-    static LFDM_HD void step(const PSet& P, const Derived& u, const K& k, S& s, const Ctl& c, double dt, bool lag,
+    static LFDM_HD void step(const PSet& P, const Derived&, const K& k, S& s, const Ctl& c, double dt, bool lag,
                              X* x) {
+        const auto& h = k.set.of(P);
         double sd, cd;
-        angles18g<G>(P, s, c.s, dt, lag, sd, cd);
-        step18g<NR, FULL, G>(P, u, k.c, k.g, s, sd, cd, c.th, c.b, dt, x);
+        angles18g<G>(h, s, c.s, dt, lag, sd, cd);
+        step18g<NR, FULL, G>(h, h.d, k.c, k.g, s, sd, cd, c.th, c.b, dt, x);
     }
     template <bool STRICT>
     static LFDM_HD void position(S& s, double dt) {
@@ -97,13 +102,18 @@ struct M18g {
     }
 };
 
+template <bool HOT>
 struct M11g {
     using S = S11g;
     using X = X11g;
-    using K = K11g;
+    struct K {
+        K11g g;
+        Params<HOT> set;
+    };
     static constexpr int kCh = M11::kCh;
     static constexpr bool kKInLds = false;
     static constexpr int kLanes = 2;
+    static constexpr bool kAhead = HOT;
     template <bool NR>
     static LFDM_HD void load(const double* st, size_t S_, int slot, S& s, K&) {
         using Rr = M11::R<NR>;
@@ -125,14 +135,16 @@ struct M11g {
     static LFDM_HD void kinit(const PSet& P, const double* o, size_t S_, const MapXY* tab, S& s, K& k) {
         K11 c;
         M11::kinit(P, o, S_, c);
-        k11g_init(P, c, s.q, k);
+        k11g_init(P, c, s.q, k.g);
+        k.set.init(P);
         walks_init<2>(P, tab, c.tqs, s.q, s.maps);
         gear_row(P, s.gear, s.row);
     }
     template <bool NR, bool FULL>
-    static LFDM_HD void step(const PSet& P, const Derived& u, const K& k, S& s, const Ctl& c, double dt, bool lag,
+    static LFDM_HD void step(const PSet& P, const Derived&, const K& k, S& s, const Ctl& c, double dt, bool lag,
                              X* x) {
-        step11g<NR, FULL>(P, u, k, s, c.s, c.th, c.b, dt, lag, x);
+        const auto& h = k.set.of(P);
+        step11g<NR, FULL>(h, h.d, k.g, s, c.s, c.th, c.b, dt, lag, x);
     }
     template <bool STRICT>
     static LFDM_HD void position(S& s, double dt) {
@@ -168,14 +180,18 @@ struct M11g {
     }
 };
 
-template <int G>
+template <int G, bool HOT>
 struct M24g {
     using S = S24g<G>;
     using X = X24g<G>;
-    using K = K24g<G>;
+    struct K {
+        K24g<G> g;
+        Params<HOT> set;
+    };
     static constexpr int kCh = M24::kCh;
     static constexpr bool kKInLds = false;
     static constexpr int kLanes = G;
+    static constexpr bool kAhead = HOT;
     static constexpr int N = S::N;
     template <bool NR>
     static LFDM_HD void load(const double* st, size_t S_, int slot, S& s, K& k) {
@@ -194,11 +210,11 @@ struct M24g {
             s.omega[j] = st[(size_t)Rr::f(i, 0) * S_ + slot];
             s.xt[j] = st[(size_t)Rr::f(i, 2) * S_ + slot];
             s.rStat[j] = st[(size_t)Rr::f(i, 4) * S_ + slot];
-            k.vsz[j] = st[(size_t)Rr::f(i, 16) * S_ + slot];
+            k.g.vsz[j] = st[(size_t)Rr::f(i, 16) * S_ + slot];
             s.xs[j] = st[(size_t)Rr::q(i, 0) * S_ + slot];
-            k.xsi[j] = st[(size_t)Rr::q(i, 1) * S_ + slot];
+            k.g.xsi[j] = st[(size_t)Rr::q(i, 1) * S_ + slot];
             s.dxs[j] = st[(size_t)Rr::q(i, 2) * S_ + slot];
-            k.lsi[j] = st[(size_t)Rr::q(i, 4) * S_ + slot];
+            k.g.lsi[j] = st[(size_t)Rr::q(i, 4) * S_ + slot];
             s.wu[j] = st[(size_t)Rr::q(i, 13) * S_ + slot];
             s.fzd[j] = st[(size_t)Rr::q(i, 20) * S_ + slot];
         }
@@ -212,14 +228,16 @@ struct M24g {
     static LFDM_HD void kinit(const PSet& P, const double* o, size_t S_, const MapXY* tab, S& s, K& k) {
         K24 c;
         M24::kinit(P, o, S_, c);
-        k24g_init<G>(P, c, s.q, k);
+        k24g_init<G>(P, c, s.q, k.g);
+        k.set.init(P);
         walks_init<G>(P, tab, c.tqs, s.q, s.maps);
         gear_row(P, s.gear, s.row);
     }
     template <bool NR, bool FULL>
-    static LFDM_HD void step(const PSet& P, const Derived& u, const K& k, S& s, const Ctl& c, double dt, bool lag,
+    static LFDM_HD void step(const PSet& P, const Derived&, const K& k, S& s, const Ctl& c, double dt, bool lag,
                              X* x) {
-        step24g<NR, FULL, G>(P, u, k, s, c.s, c.th, c.b, dt, lag, x);
+        const auto& h = k.set.of(P);
+        step24g<NR, FULL, G>(h, h.d, k.g, s, c.s, c.th, c.b, dt, lag, x);
     }
     template <bool STRICT>
     static LFDM_HD void position(S& s, double dt) {

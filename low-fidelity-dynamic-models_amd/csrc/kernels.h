@@ -28,11 +28,11 @@ constexpr int kMaxWaves11 = 4, kMaxWaves18 = 3, kMaxWaves24 = 2;
 // fleet of few wavefronts leaves SIMDs idle, so such fleets spread each vehicle over a group of lanes
 // (csrc/group.h): every lane then has one or two tires instead of four and shares the map lookups and
 // angles.  Measured per step (TMeasy fleets, microseconds; one lane / two / four):
-//   18-DOF  16,384 vehicles  7.8 / 4.0 / 2.8    32,768  8.1 / 4.2 / 4.3    65,536  8.3 / 6.3 / 7.7
-//   24-DOF  16,384 vehicles  9.9 / 5.4 / 3.6    32,768 10.3 / 5.3 / 5.1    65,536 10.3 / 8.7 / 9.8
-//   11-DOF  16,384 vehicles  4.9 / 2.6          32,768  5.5 / 2.8          65,536  5.7 / 4.0
+//   18-DOF  16,384 vehicles  7.8 / 4.0 / 2.5    32,768  8.1 / 4.2 / 4.1    65,536  8.3 / 6.1 / 7.7
+//   24-DOF  16,384 vehicles  9.9 / 5.4 / 3.2    32,768 10.3 / 5.3 / 4.9    65,536 10.3 / 8.3 / 9.8
+//   11-DOF  16,384 vehicles  4.9 / 2.4          32,768  5.5 / 2.4          65,536  5.7 / 3.9
 // So: four lanes while they make at most two wavefronts per SIMD, two lanes while they do, and one lane
-// beyond (at 131,072 18-DOF vehicles two lanes would take two rounds of 6.3 against 10.8).  The kernels are
+// beyond (at 131,072 18-DOF vehicles two lanes would take two rounds of 6.1 against 10.8).  The kernels are
 // built for the wavefronts per SIMD they make, which keeps the dispatcher from stacking two on one SIMD
 // while another is idle.  One-lane fleets of w wavefronts per SIMD, w below the model's most, run the
 // kernel built for w for the same reason.

@@ -299,13 +299,26 @@ extern "C" int group_step_run(int dof, int nr, int lanes, const double* flat, in
     *walks = group_walks(P) ? 1 : 0;
     const Run r{P, ovr, ctrl, n, rec, nsteps, dt};
     if (dof == 11 && lanes == 1) pick_tire<kern::M11, false>(r, nr, init, fin);
-    else if (dof == 11 && lanes == 2) pick_tire<kern::M11g, true>(r, nr, init, fin);
+    else if (dof == 11 && lanes == 2) pick_tire<kern::M11g<true>, true>(r, nr, init, fin);
     else if (dof == 18 && lanes == 1) pick_tire<kern::M18, false>(r, nr, init, fin);
-    else if (dof == 18 && lanes == 2) pick_tire<kern::M18g<2>, true>(r, nr, init, fin);
-    else if (dof == 18 && lanes == 4) pick_tire<kern::M18g<4>, true>(r, nr, init, fin);
+    else if (dof == 18 && lanes == 2) pick_tire<kern::M18g<2, false>, true>(r, nr, init, fin);
+    else if (dof == 18 && lanes == 4) pick_tire<kern::M18g<4, true>, true>(r, nr, init, fin);
     else if (dof == 24 && lanes == 1) pick_tire<kern::M24, false>(r, nr, init, fin);
-    else if (dof == 24 && lanes == 2) pick_tire<kern::M24g<2>, true>(r, nr, init, fin);
-    else if (dof == 24 && lanes == 4) pick_tire<kern::M24g<4>, true>(r, nr, init, fin);
+    else if (dof == 24 && lanes == 2) pick_tire<kern::M24g<2, false>, true>(r, nr, init, fin);
+    else if (dof == 24 && lanes == 4) pick_tire<kern::M24g<4, true>, true>(r, nr, init, fin);
     else return -2;
     return 0;
+}
+
+// The driver table's lookups at nt times in turn, held rows (ahead) or not: steering, throttle, braking into
+// out[nt][3].
+extern "C" void driver_lookups(const double* rows, int n, const double* times, int nt, int ascending, int ahead,
+                               double* out) {
+    const DrvRow* r = reinterpret_cast<const DrvRow*>(rows);
+    DrvWalk<false> w;
+    DrvWalk<true> wa;
+    for (int i = 0; i < nt; ++i, out += 3) {
+        if (ahead) driver_input(times[i], r, n, ascending != 0, wa, out[0], out[1], out[2]);
+        else driver_input(times[i], r, n, ascending != 0, w, out[0], out[1], out[2]);
+    }
 }

@@ -52,6 +52,40 @@ def test_lane_groups_give_the_one_lane_bits(dof, nr, n):
     np.testing.assert_array_equal(got, ref)
 
 
+@pytest.mark.parametrize("mode", ["table", "steps"])
+@pytest.mark.parametrize("dof,n", [(11, 100), (11, 32769), (18, 100), (18, 16385), (24, 100), (24, 16385)])
+def test_controls_looked_up_ahead_give_the_one_lane_bits(dof, n, mode):
+    """Driver rows and per-step controls held a step ahead (one wavefront per SIMD) and not, in three launches,
+    with horizons: 60 steps over a table of 30 rows, some out of order, the last before the end."""
+    d = os.path.join(DATA, f"{dof}dof", "HMMWV")
+    flat = lfdm_amd.params_from_json(dof, f"{d}/vehicle.json", f"{d}/tmeasy.json",
+                                     f"{d}/suspension.json" if dof == 24 else None)
+    rng = np.random.default_rng(n)
+    rows = np.column_stack([np.linspace(0.002, 0.05, 30), rng.random((30, 3)) - [0.5, 0.0, 0.0]])
+    rows[8:12, 0] = rows[[10, 8, 11, 9], 0]
+    s = SolverHalfImplicitGPU(dof, n)
+    s.construct_flat(flat, n, rows, TMeasy)
+    s.set_overrides(W.knot_fleet(n, flat, seed=n, dof=dof)["ovr"])
+    s.initialize_batch(W.initial_speed_records(n, flat, dof, seed=3))
+    if mode == "steps":
+        s.set_controls_steps(rng.random((60, 3, n)) - np.array([0.5, 0.0, 0.0])[:, None])
+    s.set_horizons(rng.integers(0, 61, n))
+    init = s.get_states()
+    with Fleet([s]) as f:
+        f.set_config(0, 64, 0, 2)  # one lane per vehicle
+        f.run(60)
+        f.synchronize()
+        ref = s.get_states()
+        s.set_states(init)
+        f.set_config(0, 64, 25, 0)
+        f.run(60)
+        f.synchronize()
+        got = s.get_states()
+    s.close()
+    assert not np.array_equal(ref, init)
+    np.testing.assert_array_equal(got, ref)
+
+
 @pytest.mark.parametrize("budget", [0, 1])
 def test_adjoint_lane_groups_give_the_one_lane_bits(budget):
     """Trajectories and gradients of fleets at the sizes where the forward's and the reverse's lanes change,

@@ -198,3 +198,41 @@ def test_jacobian_rows_equal_the_whole_steps(veh, tire, nr, walks):
                                     ctl.ctypes.data, J[full].ctypes.data) == 0
     assert np.isfinite(J[1]).all()
     np.testing.assert_array_equal(J[0], J[1])
+
+
+def driver_reference(t, rows):
+    """The reference's lookup (utils.cpp:34-56): the ends outside the table, else between the first row at or
+    after the time and the row before it."""
+    if t <= rows[0, 0]:
+        return rows[0, 1:]
+    if t >= rows[-1, 0]:
+        return rows[-1, 1:]
+    r = 1
+    while r < len(rows) - 1 and rows[r, 0] < t:
+        r += 1
+    lo, hi = rows[r - 1], rows[r]
+    return lo[1:] + ((t - lo[0]) / (hi[0] - lo[0])) * (hi[1:] - lo[1:])
+
+
+@pytest.mark.parametrize("ahead", [0, 1])
+@pytest.mark.parametrize("table", ["one row", "two rows", "double lane", "unsorted"])
+@pytest.mark.parametrize("times", ["every row many times", "several rows a step", "backwards"])
+def test_driver_rows_are_walked_to(table, times, ahead):
+    lib = ctypes.CDLL(LIB)
+    rng = np.random.Generator(np.random.PCG64(11))
+    if table == "double lane":
+        rows = np.ascontiguousarray(lfdm_amd.load_driver_file(os.path.join(DATA, "input", "double_lane4.txt")))
+    else:
+        n = {"one row": 1, "two rows": 2, "unsorted": 40}[table]
+        rows = np.column_stack([np.cumsum(rng.random(n)) + 0.3, rng.random((n, 3))])
+        if table == "unsorted":
+            rows[5:35] = rows[5 + rng.permutation(30)]
+    end = rows[-1, 0] + 1.0
+    t = np.arange(0.0, end, 0.004 if times == "every row many times" else 0.37)
+    if times == "backwards":
+        t = t[::-1]
+    t = np.ascontiguousarray(t)
+    out = np.full((len(t), 3), np.nan)
+    lib.driver_lookups(rows.ctypes.data_as(ctypes.c_void_p), len(rows), t.ctypes.data_as(ctypes.c_void_p), len(t),
+                       int(times != "backwards"), ahead, out.ctypes.data_as(ctypes.c_void_p))
+    np.testing.assert_array_equal(out, np.array([driver_reference(x, rows) for x in t]))
