@@ -15,6 +15,7 @@ struct S11 {
     double xe[2], ye[2], xedot[2], yedot[2], omega[2];
     double x, y, u, v, psi, wz, udot, crank;
     int gear;
+    unsigned places = kNoPlaces;
 };
 
 // Quantities of the last right-hand side that the full state record also holds.
@@ -106,7 +107,7 @@ LFDM_HD void step11(const PSet& P, const Derived& u, const K11& k, S11& s, doubl
     }
     // computePowertrainRHS (dof11.cpp:607-749)
     double torque_t, dcrank;
-    powertrain_torque<STRICT>(P, u, k.tqs, throttle, s.u, 0.5 * (s.omega[0] + s.omega[1]), s.crank, s.gear, torque_t,
+    powertrain_torque<STRICT>(P, u, k.tqs, throttle, s.u, 0.5 * (s.omega[0] + s.omega[1]), s.crank, s.gear, s.places, torque_t,
                               dcrank);
     // differentialSplit between the axles (dof11.cpp:271-311): 4WD splits with the bias rule
     // (rear axle in the "left" slot), else whichWheels picks the driven axle

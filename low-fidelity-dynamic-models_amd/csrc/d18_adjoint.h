@@ -40,30 +40,17 @@ LFDM_HD void k18b_zero(K18b& b) {
     b.denom = b.A1A2 = b.A1A3 = b.A3sq = b.qy1 = b.qy2 = b.jz = b.tqs = b.maxBrake = 0.0;
 }
 
-// Slope of a clamped piecewise-linear map at x on the segment map_y uses (0 outside the knots).
-LFDM_HD double map_slope(const Map& m, double x) {
-    const int n = m.n;
-    if (x <= m.e[0].x || x >= m.e[n - 1].x) return 0.0;
-    int r = 0;
-    for (int k = 1; k < n - 1; ++k) r += (m.e[k].x < x) ? 1 : 0;
-    r += 1;
-    return fdiv(m.e[r].y - m.e[r - 1].y, m.e[r].x - m.e[r - 1].x);
-}
-
-// map_y(m, x) and the slope of the segment it uses (0 where it clamps), from one scan of the knots.
+// map_y(m, x) and the slope of the segment it uses (0 where it clamps).  The adjoint scans: its kernel, one
+// wavefront per SIMD on 512 registers, ran 1-2 % slower walking (find_segment) from the step after's places.
 LFDM_HD double map_y_slope(const Map& m, double x, double& slope) {
-    const int n = m.n;
     slope = 0.0;
     if (x <= m.e[0].x) return m.e[0].y;
-    if (x >= m.e[n - 1].x) return m.e[n - 1].y;
-    int r = 0;
-    for (int k = 1; k < n - 1; ++k) r += (m.e[k].x < x) ? 1 : 0;
-    r += 1;
-    const MapXY L = m.e[r - 1];
-    const MapXY R = m.e[r];
-    slope = fdiv(R.y - L.y, R.x - L.x);
-    const double mbar = fdiv(x - L.x, R.x - L.x);
-    return L.y + mbar * (R.y - L.y);
+    if (x >= m.e[m.n - 1].x) return m.e[m.n - 1].y;
+    int r;
+    const Segment g = scan_segment(m, x, r);
+    slope = fdiv(g.R.y - g.L.y, g.R.x - g.L.x);
+    const double mbar = fdiv(x - g.L.x, g.R.x - g.L.x);
+    return g.L.y + mbar * (g.R.y - g.L.y);
 }
 
 // d sineStep(x, 1, 1, 1.5, 0) / dx; the cosine of the turn fraction v = (x - 1) / dx as the sine a
@@ -401,7 +388,7 @@ LFDM_HD void powertrain4_adj(const PSet& P, const Derived& u, double tqs, double
                              double braking, double vel_u, double crank, int gear, const double* omega,
                              const double* fx, const double* rStat, const double* My, PtBars& B) {
     const double osum = omega[0] + omega[1] + omega[2] + omega[3];
-    const double gr = pick(P.gears, P.ngears, gear);
+    const double gr = P.gears[gear_index(gear, P.ngears)];
     // ---- forward recompute ----
     double torque_t, torque_in = 0, torque_out = 0, sr0 = 0, q = 0, cf = 1, tr = 0, cfs = 0, trs = 0;
     bool active = false, rev = false, clip = false;
@@ -476,8 +463,9 @@ LFDM_HD void powertrain4_adj(const PSet& P, const Derived& u, double tqs, double
         ttb = tfb;
     if (clip) ttb = 0;
     // drive torque at w_dt: tqs * T(w) * throttle + L(w)
-    double Ts;
-    const double Tw = map_y_slope(P.torque, w_dt, Ts), Ls = map_slope(P.losses, w_dt);
+    double Ts, Ls;
+    const double Tw = map_y_slope(P.torque, w_dt, Ts);
+    map_y_slope(P.losses, w_dt, Ls);
     const double rgr = frcp(gr);
     if (P.tcbool) {
         const double omega_in = crank;

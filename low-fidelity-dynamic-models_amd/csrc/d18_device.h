@@ -17,6 +17,7 @@ struct S18 {
     double xe[4], ye[4], xedot[4], yedot[4], omega[4];
     double x, y, u, v, psi, wz, phi, wx, udot, vdot, crank;
     int gear;
+    unsigned places = kNoPlaces;
 };
 
 // Quantities of the last right-hand side that the full state record also holds.
@@ -202,7 +203,7 @@ LFDM_HD void step18(const PSet& P, const Derived& u, const K18& k, S18& s, doubl
     }
     // computePowertrainRHS
     double dOm[4], eng[4], dcrank;
-    powertrain4<STRICT>(P, u, k.tqs, k.maxBrake, throttle, braking, s.u, s.crank, s.gear, s.omega, fx, rStat, My, dOm, eng,
+    powertrain4<STRICT>(P, u, k.tqs, k.maxBrake, throttle, braking, s.u, s.crank, s.gear, s.places, s.omega, fx, rStat, My, dOm, eng,
                 dcrank);
     // tireToVehTransform (front tires only)
 #pragma unroll

@@ -116,7 +116,7 @@ LFDM_HD void powertrain_group_adj(const PSet& P, const Derived& u, const K18& c,
             drive = drive_torque<false>(P, tqs, throttle, w_dt);
         }
         Tw = map_y_slope(P.torque, w_dt, Ts);
-        Ls = map_slope(P.losses, w_dt);
+        map_y_slope(P.losses, w_dt, Ls);
     } else if constexpr (G == 4) {
         double m, ys;
         const double y = walk_slope(w.maps.a, La, Ra, q < 2 ? sr : w_dt, m, ys);

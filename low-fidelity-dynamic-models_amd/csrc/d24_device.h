@@ -24,6 +24,7 @@ struct S24 {
     double x, y, u, v, w, psi, phi, theta, wx, wy, wz;
     double udot, vdot, wdot, wxdot, wydot, wzdot, crank;
     int gear;
+    unsigned places = kNoPlaces;
 };
 
 // Quantities of the last right-hand side that the full state record also holds.
@@ -193,7 +194,7 @@ LFDM_HD void step24(const PSet& P, const Derived& u, K24& k, S24& s, double stee
     }
     // computePowertrainRHS (dof24.cpp:1338-1509)
     double dOm[4], eng[4], dcrank;
-    powertrain4<STRICT>(P, u, k.tqs, k.maxBrake, throttle, braking, s.u, s.crank, s.gear, s.omega, fx, s.rStat, My, dOm, eng,
+    powertrain4<STRICT>(P, u, k.tqs, k.maxBrake, throttle, braking, s.u, s.crank, s.gear, s.places, s.omega, fx, s.rStat, My, dOm, eng,
                 dcrank);
 #pragma unroll
     for (int i = 0; i < 4; ++i) {

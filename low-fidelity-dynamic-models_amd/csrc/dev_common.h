@@ -376,27 +376,41 @@ LFDM_HD double sine_step(double x, double x1, double y1, double x2, double y2) {
     return y1 + fdiv(dy * (x - x1), dx) - fdiv(dy, k2Pi) * sin_2pi_unit(fdiv(x - x1, dx));
 }
 
-// Clamped piecewise-linear lookup (utils.cpp:109-125). `m` is wave-uniform, so the knot scan
-// runs on scalar loads; the interval index counts knots strictly below x, which is exactly
-// std::lower_bound's answer on a sorted map.  Branch-free: the segment the scan picks is
-// interpolated for every x (the first segment at or below the first knot, the last at or above the
-// last knot; a one-knot map reads the zero entry after it, whose result is never selected) and the
-// end values are selected outside the knots, so a wavefront takes no divergent branch and its
-// scalar loads are not held behind one.
+// A map's segment of an abscissa: the knots r - 1 and r around it.
+struct Segment {
+    MapXY L, R;
+};
+
+// The segment the scan picks: 1 <= r <= n - 1, r - 1 the knots but the first and last strictly below x, which
+// is std::lower_bound's answer on a sorted map.  `m` is wave-uniform, so the knots are scalar loads.
+LFDM_HD Segment scan_segment(const Map& m, double x, int& r) {
+    r = 1;
+    for (int k = 1; k < m.n - 1; ++k) r += (m.e[k].x < x) ? 1 : 0;
+    return {m.e[r - 1], m.e[r]};
+}
+
+// Clamped piecewise-linear lookup (utils.cpp:109-125) on the segment of x.  Branch-free: the segment is
+// interpolated for every x (the first segment at or below the first knot, the last at or above the last knot; a
+// one-knot map reads the zero entry after it, whose result is never selected) and the end values are selected
+// outside the knots, so a wavefront takes no divergent branch and its scalar loads are not held behind one.
+// Ordinates are multiplied by sy (by 1.0: exact).
+template <bool STRICT>
+LFDM_HD double map_y_on(const Map& m, const Segment& g, double x, double sy) {
+    const double ly = g.L.y * sy, ry = g.R.y * sy;
+    // a division by the segment's width: the reference's quotient is exact at the knots (a car at
+    // rest sits on one, where any residue would feed the torque converter's own feedback and never
+    // rest), which a reciprocal width would not
+    const double mbar = xdiv<STRICT>(x - g.L.x, g.R.x - g.L.x);
+    const double y = ly + mbar * (ry - ly);
+    const MapXY F = m.e[0], B = m.e[m.n - 1];
+    return x <= F.x ? F.y * sy : (x >= B.x ? B.y * sy : y);
+}
+
 template <bool STRICT>
 LFDM_HD double map_y(const Map& m, double x) {
-    const int n = m.n;
-    int r = 0;
-    for (int k = 1; k < n - 1; ++k) r += (m.e[k].x < x) ? 1 : 0;
-    r += 1;
-    const MapXY L = m.e[r - 1];
-    const MapXY R = m.e[r];
-    // a division in both forms: a map through the origin gives exactly 0 at 0 (the powertrain's losses at
-    // rest), which a reciprocal width would not
-    const double mbar = xdiv<STRICT>(x - L.x, R.x - L.x);
-    const double y = L.y + mbar * (R.y - L.y);
-    const MapXY F = m.e[0], B = m.e[n - 1];
-    return x <= F.x ? F.y : (x >= B.x ? B.y : y);
+    int r;
+    const Segment g = scan_segment(m, x, r);
+    return map_y_on<STRICT>(m, g, x, 1.0);
 }
 
 // Same lookup on a map whose abscissae are scaled by sx and ordinates by sy1 then sy2
@@ -414,6 +428,38 @@ LFDM_HD double map_y_scaled(const Map& m, double x, double sx, double sy1, doubl
     const double y = ly + mbar * (ry - ly);
     const MapXY F = m.e[0], B = m.e[n - 1];
     return x <= F.x * sx ? F.y * sy1 * sy2 : (x >= B.x * sx ? B.y * sy1 * sy2 : y);
+}
+
+// Where a vehicle's last lookups on its powertrain maps ended: byte id holds map id's segment, r - 1, or
+// kNoPlace.
+enum { kMapCf = 0, kMapTr = 1, kMapTorque = 2, kMapLosses = 3 };
+constexpr unsigned kNoPlace = 255u, kNoPlaces = ~0u;
+
+// scan_segment by walking from the place of the last lookup: two compares, since a step later the abscissa
+// nearly always lies on the same segment.  A vehicle without a place, and a map whose abscissae do not ascend,
+// is scanned: 37 knots for the HMMWV's four maps, each a scalar load waited for.  Per step, scanned -> walked:
+// 18-DOF 71.9 -> 69.8 us (1,000,000 vehicles), 11.4 -> 10.9 (100,003), TMeasyNr 38.5 -> 37.0 (300,000); 11-DOF
+// 27.0 -> 26.2 (600,000); 24-DOF 27.9 -> 27.2 (250,000).  The segments are loaded where they are used: asked for
+// together at the powertrain's start they held registers the 24-DOF step has not (28.9).
+LFDM_HD Segment find_segment(const Map& m, double x, int id, unsigned& places) {
+    const unsigned p = places >> (8 * id) & 255u;
+    Segment g;
+    int r;
+    if (p == kNoPlace) {
+        g = scan_segment(m, x, r);
+        if (!m.sorted) return g;
+    } else {
+        r = (int)p + 1;
+        g = {m.e[p], m.e[r]};
+        for (;;) {
+            const bool down = r > 1 && !(g.L.x < x), up = r < m.n - 1 && g.R.x < x;
+            if (!(down || up)) break;
+            r += up ? 1 : -1;
+            g = {m.e[r - 1], m.e[r]};
+        }
+    }
+    places += ((unsigned)(r - 1) - p) << (8 * id);
+    return g;
 }
 
 // Where the last lookup in a driver table ended: its row, and, with AHEAD, the rows around it and the table's
@@ -465,12 +511,8 @@ LFDM_HD void driver_input(double t, const DrvRow* __restrict__ rows, int n, bool
     }
 }
 
-// Gear-indexed reads by a per-lane gear over a wave-uniform table (select chain, no memory).
-LFDM_HD double pick(const double* tab, int n, int i) {
-    double v = tab[0];
-    for (int k = 1; k < n; ++k) v = (i == k) ? tab[k] : v;
-    return v;
-}
+// The gear whose row a lane reads: the reference's gear, the first where a record holds none of the set's.
+LFDM_HD int gear_index(int gear, int ngears) { return (unsigned)gear < (unsigned)ngears ? gear : 0; }
 
 }  // namespace dev
 }  // namespace lfdm

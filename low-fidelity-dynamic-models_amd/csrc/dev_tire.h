@@ -390,25 +390,29 @@ LFDM_HD void diff_split(double torque, double sl, double sr, double& tl, double&
 }
 
 // driveTorque (dof18.cpp:15-42, dof11.cpp:15-42, dof24.cpp:92-119) with the per-vehicle torque
-// scale tqs on the map ordinates.
+// scale tqs on the map ordinates.  A torque map scaled by the throttle is scanned.
+template <bool STRICT>
+LFDM_HD double drive_torque(const PSet& P, double tqs, double throttle, double w, unsigned& places) {
+    const double losses = map_y_on<STRICT>(P.losses, find_segment(P.losses, w, kMapLosses, places), w, 1.0);
+    if (P.throttleMod) return map_y_scaled<STRICT>(P.torque, w, throttle, tqs, throttle) + losses;
+    return map_y_on<STRICT>(P.torque, find_segment(P.torque, w, kMapTorque, places), w, tqs) * throttle + losses;
+}
+
 template <bool STRICT>
 LFDM_HD double drive_torque(const PSet& P, double tqs, double throttle, double w) {
-    if (P.throttleMod) {
-        const double tq = map_y_scaled<STRICT>(P.torque, w, throttle, tqs, throttle);
-        return tq + map_y<STRICT>(P.losses, w);
-    }
-    const double tq = map_y_scaled<STRICT>(P.torque, w, 1.0, tqs, 1.0);
-    return tq * throttle + map_y<STRICT>(P.losses, w);
+    unsigned places = kNoPlaces;
+    return drive_torque<STRICT>(P, tqs, throttle, w, places);
 }
 
 // The part of computePowertrainRHS (dof18.cpp:675-800, dof24.cpp:1338-1462, dof11.cpp:607-720) ahead of the axles: torque
 // converter or slaved crank and the gear shift for the next step, from the wheels' mean speed.
-// Updates crank (without a converter) and gear; returns the shaft torque and dcrank.
+// Updates crank (without a converter), gear and the places on the maps; returns the shaft torque and dcrank.
 template <bool STRICT>
 LFDM_HD void powertrain_torque(const PSet& P, const Derived& u, double tqs, double throttle, double vel_u, double mean,
-                               double& crank, int& gear, double& torque_t, double& dcrank) {
+                               double& crank, int& gear, unsigned& places, double& torque_t, double& dcrank) {
     dcrank = 0.0;
-    const double gr = pick(P.gears, P.ngears, gear);
+    const int gi = gear_index(gear, P.ngears);
+    const double gr = P.gears[gi];
     double shift_w;
     // the quotients by the gear ratio stay divisions in the fast form too: the converter's speed ratio
     // omega_out / crank is exactly 1 at a crank speed set from the same quotient, and the model's
@@ -426,33 +430,27 @@ LFDM_HD void powertrain_torque(const PSet& P, const Derived& u, double tqs, doub
             }
             if (sr < 0) sr = 0;
         }
-        const double cf = map_y<STRICT>(P.cfmap, sr);
-        const double tr = map_y<STRICT>(P.trmap, sr);
+        const double cf = map_y_on<STRICT>(P.cfmap, find_segment(P.cfmap, sr, kMapCf, places), sr, 1.0);
+        const double tr = map_y_on<STRICT>(P.trmap, find_segment(P.trmap, sr, kMapTr, places), sr, 1.0);
         const double q = xdiv<STRICT>(omega_in, cf);
         double torque_in = -(q * q);
         if (rev) torque_in = -torque_in;
         const double torque_out = rev ? -torque_in : -tr * torque_in;
         torque_t = xdiv<STRICT>(torque_out, gr);
         if (vel_u < 1e-9 && torque_t < 0) torque_t = 0;
-        dcrank = u.inv_ci * (drive_torque<STRICT>(P, tqs, throttle, crank) + torque_in);
+        dcrank = u.inv_ci * (drive_torque<STRICT>(P, tqs, throttle, crank, places) + torque_in);
         shift_w = omega_out;
     } else {
         crank = xdiv<STRICT>(mean, gr);
-        torque_t = xdiv<STRICT>(drive_torque<STRICT>(P, tqs, throttle, crank), gr);
+        torque_t = xdiv<STRICT>(drive_torque<STRICT>(P, tqs, throttle, crank, places), gr);
         if (vel_u < 1e-9 && torque_t < 0) torque_t = 0;
         shift_w = crank;
     }
-    {
-        double up = P.shift[0].y, dn = P.shift[0].x;
-        for (int g = 1; g < P.ngears; ++g) {
-            up = (gear == g) ? P.shift[g].y : up;
-            dn = (gear == g) ? P.shift[g].x : dn;
-        }
-        if (shift_w > up) {
-            if (gear < P.ngears - 1) gear++;
-        } else if (shift_w < dn) {
-            if (gear > 0) gear--;
-        }
+    const MapXY shift = P.shift[gi];
+    if (shift_w > shift.y) {
+        if (gear < P.ngears - 1) gear++;
+    } else if (shift_w < shift.x) {
+        if (gear > 0) gear--;
     }
 }
 
@@ -477,11 +475,11 @@ LFDM_HD void axle_torques(const PS& P, double torque_t, double& tf, double& trr)
 template <bool STRICT>
 LFDM_HD void powertrain4(const PSet& P, const Derived& u, double tqs, double maxBrake,
                                             double throttle, double braking, double vel_u, double& crank, int& gear,
-                                            const double* omega, const double* fx, const double* rStat,
-                                            const double* My, double* dOm, double* eng, double& dcrank) {
+                                            unsigned& places, const double* omega, const double* fx,
+                                            const double* rStat, const double* My, double* dOm, double* eng, double& dcrank) {
     double torque_t, tf, trr;
     const double osum = omega[0] + omega[1] + omega[2] + omega[3];
-    powertrain_torque<STRICT>(P, u, tqs, throttle, vel_u, 0.25 * osum, crank, gear, torque_t, dcrank);
+    powertrain_torque<STRICT>(P, u, tqs, throttle, vel_u, 0.25 * osum, crank, gear, places, torque_t, dcrank);
     axle_torques(P, torque_t, tf, trr);
     diff_split<STRICT>(tf, omega[0], omega[1], eng[0], eng[1]);
     diff_split<STRICT>(trr, omega[2], omega[3], eng[2], eng[3]);

@@ -57,7 +57,6 @@ LFDM_HD void group_tires(const double* v, double* all) {
 // and two compares instead of a scan of every knot by scalar loads and a vector load of the segment found
 // (for the HMMWV's four maps, 37 knots).  On ascending abscissae the walk ends at the interval the scan
 // counts to (map_y), for any start.
-enum { kMapCf = 0, kMapTr = 1, kMapTorque = 2, kMapLosses = 3 };
 constexpr int kGroupMaps = 4;
 constexpr int kGroupMapEntries = kGroupMaps * kMaxMap;  // LDS entries of one wavefront
 
@@ -115,20 +114,19 @@ LFDM_HD void walks_init(const PSet& P, const MapXY* tab, double tqs, int q, Walk
     if (G == 2) walk_init(P, tab, tqs, 2 + q, w.b);
 }
 
-// The current gear's ratio, the ratio's reciprocal as fdiv refines it, and shift speeds.
+// The current gear's ratio, the ratio's reciprocal as fdiv refines it, and shift speeds; the places of a
+// vehicle whose set the walk does not serve.
 struct GearRow {
     double ratio, rcp, up, down;
+    unsigned places = kNoPlaces;
 };
 
 LFDM_HD void gear_row(const PSet& P, int gear, GearRow& g) {
-    g.ratio = pick(P.gears, P.ngears, gear);
+    const int i = gear_index(gear, P.ngears);
+    g.ratio = P.gears[i];
     g.rcp = fdiv_rcp(g.ratio);
-    g.up = P.shift[0].y;
-    g.down = P.shift[0].x;
-    for (int i = 1; i < P.ngears; ++i) {
-        g.up = (gear == i) ? P.shift[i].y : g.up;
-        g.down = (gear == i) ? P.shift[i].x : g.down;
-    }
+    g.up = P.shift[i].y;
+    g.down = P.shift[i].x;
 }
 
 // Sets the walk does not serve (a map that does not ascend, or a torque map scaled by the throttle)
@@ -194,7 +192,7 @@ LFDM_HD void powertrain_group(const PS& P, const Derived& u, double tqs, double 
                               int q, bool walks, Walks<G>& w, GearRow& g, double& crank, int& gear,
                               double& torque_t, double& dcrank) {
     if (!walks) {
-        powertrain_torque<false>(full_set(P), u, tqs, throttle, vel_u, mean, crank, gear, torque_t, dcrank);
+        powertrain_torque<false>(full_set(P), u, tqs, throttle, vel_u, mean, crank, gear, g.places, torque_t, dcrank);
         return;
     }
     const MapXY La = w.a.e[w.a.r - 1], Ra = w.a.e[w.a.r];

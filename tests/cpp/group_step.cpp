@@ -322,3 +322,16 @@ extern "C" void driver_lookups(const double* rows, int n, const double* times, i
         else driver_input(times[i], r, n, ascending != 0, w, out[0], out[1], out[2]);
     }
 }
+
+// Lookups on one map at nx abscissae in turn, each walking from the last one's place: the ordinates times sy.
+extern "C" void map_lookups(const double* knots, int n, int sorted, const double* x, int nx, double sy, int id,
+                            double* out) {
+    Map m{};
+    m.n = n;
+    m.sorted = sorted;
+    for (int i = 0; i < n; ++i) m.e[i] = {knots[2 * i], knots[2 * i + 1]};
+    unsigned places = kNoPlaces;
+    for (int i = 0; i < nx; ++i) out[i] = map_y_on<true>(m, find_segment(m, x[i], id, places), x[i], sy);
+}
+
+extern "C" int gear_row_of(int gear, int ngears) { return gear_index(gear, ngears); }

@@ -236,3 +236,43 @@ def test_driver_rows_are_walked_to(table, times, ahead):
     lib.driver_lookups(rows.ctypes.data_as(ctypes.c_void_p), len(rows), t.ctypes.data_as(ctypes.c_void_p), len(t),
                        int(times != "backwards"), ahead, out.ctypes.data_as(ctypes.c_void_p))
     np.testing.assert_array_equal(out, np.array([driver_reference(x, rows) for x in t]))
+
+
+def map_reference(x, m, sy):
+    """The reference's lookup (utils.cpp:109-125) as a scan of every knot, ordinates times sy."""
+    if x <= m[0, 0]:
+        return m[0, 1] * sy
+    if x >= m[-1, 0]:
+        return m[-1, 1] * sy
+    r = 1 + int((m[1:-1, 0] < x).sum())
+    (lx, ly), (rx, ry) = m[r - 1], m[r]
+    return ly * sy + (x - lx) / (rx - lx) * (ry * sy - ly * sy)
+
+
+@pytest.mark.parametrize("id", [0, 3])
+@pytest.mark.parametrize("knots", ["1", "2", "3", "48", "repeated", "unsorted"])
+def test_map_walk_gives_the_scanned_value(knots, id):
+    """Walks up, down and over many knots, to every knot itself and past both ends, and over a NaN."""
+    lib = ctypes.CDLL(LIB)
+    lib.map_lookups.argtypes = [ctypes.c_void_p, ctypes.c_int, ctypes.c_int, ctypes.c_void_p, ctypes.c_int,
+                                ctypes.c_double, ctypes.c_int, ctypes.c_void_p]
+    rng = np.random.Generator(np.random.PCG64(5))
+    n = int(knots) if knots.isdigit() else 20
+    m = np.column_stack([np.cumsum(rng.random(n)) - 2.0, rng.normal(size=n)])
+    if knots == "repeated":
+        m[7:10, 0] = m[7, 0]
+    if knots == "unsorted":
+        m[1:-1] = m[1 + rng.permutation(n - 2)]
+    near = np.sort(np.concatenate([m[:, 0], rng.uniform(m[0, 0] - 1, m[-1, 0] + 1, 400)]))
+    x = np.concatenate([near, near[::-1], rng.permutation(near), [np.nan], rng.permutation(near)])
+    out = np.full(len(x), -1.0)
+    ptr = lambda a: a.ctypes.data  # noqa: E731
+    m = np.ascontiguousarray(m)
+    lib.map_lookups(ptr(m), n, int(knots != "unsorted"), ptr(x), len(x), 0.7, id, ptr(out))
+    # (on the repeated knots the segment has no width and no abscissa lies strictly inside it)
+    np.testing.assert_array_equal(out, np.array([np.nan if np.isnan(v) else map_reference(v, m, 0.7) for v in x]))
+
+
+def test_gear_outside_the_set_reads_the_first_row():
+    lib = ctypes.CDLL(LIB)
+    assert [lib.gear_row_of(g, 4) for g in (-(1 << 31), -1, 0, 3, 4, 9)] == [0, 0, 0, 3, 0, 0]
