@@ -335,3 +335,12 @@ extern "C" void map_lookups(const double* knots, int n, int sorted, const double
 }
 
 extern "C" int gear_row_of(int gear, int ngears) { return gear_index(gear, ngears); }
+
+// The sine-step weights of pairs, together (out[4 i], out[4 i + 1]) and one by one (out[4 i + 2], out[4 i + 3]).
+extern "C" void weight_pairs(const double* x, const double* y, int n, double* out) {
+    for (int i = 0; i < n; ++i, out += 4) {
+        sine_step_weights<false>(x[i], y[i], out[0], out[1]);
+        out[2] = sine_step_weight<false>(x[i]);
+        out[3] = sine_step_weight<false>(y[i]);
+    }
+}

@@ -276,3 +276,13 @@ def test_map_walk_gives_the_scanned_value(knots, id):
 def test_gear_outside_the_set_reads_the_first_row():
     lib = ctypes.CDLL(LIB)
     assert [lib.gear_row_of(g, 4) for g in (-(1 << 31), -1, 0, 3, 4, 9)] == [0, 0, 0, 3, 0, 0]
+
+
+def test_sine_step_weights_of_a_pair():
+    """Below, inside, above and at the ends of the blend, in every combination, and NaN."""
+    lib = ctypes.CDLL(LIB)
+    v = np.array([0.0, 0.5, 1.0, np.nextafter(1.0, 2), 1.1, 1.25, 1.4, np.nextafter(1.5, 1), 1.5, 2.0, np.inf, np.nan])
+    x, y = (np.ascontiguousarray(a.ravel()) for a in np.meshgrid(v, v))
+    out = np.full((len(x), 4), -1.0)
+    lib.weight_pairs(*(a.ctypes.data_as(ctypes.c_void_p) for a in (x, y)), len(x), out.ctypes.data_as(ctypes.c_void_p))
+    np.testing.assert_array_equal(out[:, :2], out[:, 2:])
