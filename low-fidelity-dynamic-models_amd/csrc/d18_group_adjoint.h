@@ -443,7 +443,11 @@ LFDM_HD void load_record_g(const double* st, size_t S, int slot, S18g<G>& s) {
 
 // adj_forward_lane on a group.  A step's position update comes with the next step's angles, so the positions
 // of step j are written by step j + 1 (the last step's after the loop).
-template <int G>
+// HOT: the set's parameters in registers (HotSet).  On four lanes, which have the registers, the controls are
+// loaded a step ahead of their use.  Per step 2.95 -> 2.83 us (1,000 vehicles), 3.30 -> 3.13 (16,384), 4.90 -> 4.62
+// (32,768, two wavefronts per SIMD: controls only).  The reverse sweep has no room for either: with HotSet 6.33 ->
+// 6.86 (1,000), with the next tape row held 6.53.
+template <int G, bool HOT>
 LFDM_HD void adj_forward_group(const AdjLaunch& L, int slot, int q, const PSet& P, const MapXY* tab) {
     const size_t S = (size_t)L.S, N = (size_t)L.n_user;
     S18g<G> s;
@@ -455,33 +459,46 @@ LFDM_HD void adj_forward_group(const AdjLaunch& L, int slot, int q, const PSet& 
     k18g_init<G>(P, c, q, k);
     walks_init<G>(P, tab, c.tqs, q, s.maps);
     gear_row(P, s.gear, s.row);
+    Params<HOT> set;
+    set.init(P);
+    const auto& h = set.of(P);
     const int user = L.slot_user[slot];
     const int uv = user >= 0 ? user : 0;
     const bool writes = user >= 0 && q == 0;
     const int jt = L.fwd_tape_lo * L.K < L.nsteps ? L.fwd_tape_lo * L.K : L.nsteps;
     int seg = 0, jj = 0;  // segment of step j and the step's index in it
+    constexpr bool kAhead = G == 4;
+    const double* ctl = L.ctrl + uv;
+    double next[3] = {ctl[0], ctl[N], ctl[2 * N]};
     for (int j = 0; j < L.nsteps; ++j) {
-        const double* ctl = L.ctrl + (size_t)j * 3 * N + uv;
-        const double steering = ctl[0], throttle = ctl[N], braking = ctl[2 * N];
+        const double steering = next[0], throttle = next[1], braking = next[2];
+        if (kAhead && j + 1 < L.nsteps) {
+            ctl += 3 * N;
+            next[0] = ctl[0]; next[1] = ctl[N]; next[2] = ctl[2 * N];
+        }
         double sd, cd;
-        angles18g<G>(P, s, steering, L.dt, j > 0, sd, cd);
+        angles18g<G>(h, s, steering, L.dt, j > 0, sd, cd);
         if (writes && j > 0) {
             L.xy[(size_t)(j - 1) * 2 * N + user] = s.x;
             L.xy[((size_t)(j - 1) * 2 + 1) * N + user] = s.y;
         }
         if (jj == 0) pack_g<G>(s, L.ckpt + (size_t)seg * kCarried * S + slot, S);
         if (j < jt) {
-            step18g<false, false, G>(P, P.d, c, k, s, sd, cd, throttle, braking, L.dt, nullptr);
+            step18g<false, false, G>(h, h.d, c, k, s, sd, cd, throttle, braking, L.dt, nullptr);
         } else {
             double* row = tape_row(L, seg - L.fwd_tape_lo, jj, slot);
             tape_put_state_g<G>(s, row);
             TireOut18g<G> to;
-            step18g<false, false, G, true>(P, P.d, c, k, s, sd, cd, throttle, braking, L.dt, nullptr, &to);
+            step18g<false, false, G, true>(h, h.d, c, k, s, sd, cd, throttle, braking, L.dt, nullptr, &to);
             tape_put_tires_g<G>(to, q, row);
         }
         if (++jj == L.K) {
             jj = 0;
             ++seg;
+        }
+        if (!kAhead && j + 1 < L.nsteps) {
+            ctl += 3 * N;
+            next[0] = ctl[0]; next[1] = ctl[N]; next[2] = ctl[2 * N];
         }
     }
     double sp, cp;

@@ -31,7 +31,7 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(W, W))
     int slot, q;
     const PSet* P;
     if (!group_lane<G>(L, tab, slot, q, P)) return;
-    adj_forward_group<G>(L, slot, q, *P, tab);
+    adj_forward_group<G, W == 1>(L, slot, q, *P, tab);
 }
 
 // The constants and their adjoints lie in LDS once per vehicle: in registers they would take 88 of a lane's

@@ -153,7 +153,7 @@ void on_lanes(const PSet& P, F body) {
 template <int G>
 void adjoint_group(const PSet& P, AdjLaunch L, int nseg, int group) {
     for (int v = 0; v < L.n_user; ++v)
-        on_lanes<G>(P, [&](int q, const MapXY* tab) { adj_forward_group<G>(L, v, q, P, tab); });
+        on_lanes<G>(P, [&](int q, const MapXY* tab) { adj_forward_group<G, G == 4>(L, v, q, P, tab); });
     for (int hi = nseg; hi > 0; hi -= group) {
         L.seg_hi = hi;
         L.seg_lo = hi - group > 0 ? hi - group : 0;
