@@ -35,8 +35,8 @@ constexpr int kThreads = 256;
 
 static_assert(sizeof(K18) % 16 == 8 && sizeof(K18b) % 16 == 8, "odd number of doubles per lane in LDS");
 
-template <int W>
-__global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(W, W))) void adj_forward(AdjLaunch L) {
+// Two waves per SIMD: fleets of no more than one run on lane groups (choose_kernel).
+__global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2, 2))) void adj_forward(AdjLaunch L) {
     const int slot = blockIdx.x * blockDim.x + threadIdx.x;
     const int wave = uniform(slot >> 6);
     if (wave * kWave >= L.S) return;
@@ -81,12 +81,9 @@ hipError_t launch_step_jacobian(const AdjLaunch& L, hipStream_t stream) {
     return hipGetLastError();
 }
 
-hipError_t launch_adj_forward(const AdjLaunch& L, int waves_per_simd, hipStream_t stream) {
+hipError_t launch_adj_forward(const AdjLaunch& L, hipStream_t stream) {
     if (L.S <= 0 || L.nsteps <= 0) return hipSuccess;
-    if (waves_per_simd == 1)
-        hipLaunchKernelGGL(adj_forward<1>, (L.S + kThreads - 1) / kThreads, kThreads, 0, stream, L);
-    else
-        hipLaunchKernelGGL(adj_forward<2>, (L.S + kThreads - 1) / kThreads, kThreads, 0, stream, L);
+    hipLaunchKernelGGL(adj_forward, (L.S + kThreads - 1) / kThreads, kThreads, 0, stream, L);
     return hipGetLastError();
 }
 

@@ -140,9 +140,8 @@ struct AdjLaunch {
 constexpr int kJacRows = 21;
 constexpr int kJacCols = kJacRows + 3;
 
-// waves_per_simd 1 or 2: register budget of the forward kernel (1 when the fleet fills at most one
-// wavefront per SIMD, so the step runs without spills).
-hipError_t launch_adj_forward(const AdjLaunch& L, int waves_per_simd, hipStream_t stream);
+// The forward pass: one lane per vehicle on fleets of more than one wavefront per SIMD, else on lane groups.
+hipError_t launch_adj_forward(const AdjLaunch& L, hipStream_t stream);
 hipError_t launch_adj_forward_group(const AdjLaunch& L, KernelChoice c, hipStream_t stream);
 hipError_t launch_adj_reverse_group(const AdjLaunch& L, int lanes, hipStream_t stream);
 hipError_t launch_adj_recompute(const AdjLaunch& L, hipStream_t stream);

@@ -1411,11 +1411,9 @@ int lfdm_adjoint_forward(lfdm_solver* h, int nsteps, int checkpoint_every, const
     AdjLaunch L = adj_launch(h);
     L.xy = dxy;
     L.fwd_tape_lo = (int)nseg - G;
-    // a fleet of at most one wavefront per SIMD gets the whole register file per lane
-    const int waves = (size_t)h->S / kWave <= (size_t)simds ? 1 : 2;
     HIPCHK(hipEventRecord(h->ev0, h->stream));
     const KernelChoice fc = choose_kernel(18, h->S, simds, false);
-    hipError_t e = fc.lanes > 1 ? launch_adj_forward_group(L, fc, h->stream) : launch_adj_forward(L, waves, h->stream);
+    hipError_t e = fc.lanes > 1 ? launch_adj_forward_group(L, fc, h->stream) : launch_adj_forward(L, h->stream);
     if (e != hipSuccess) return fail(LFDM_E_HIP, std::string("adjoint forward launch failed: ") + hipGetErrorString(e));
     HIPCHK(hipEventRecord(h->ev1, h->stream));
     h->timed = true;
@@ -1530,7 +1528,7 @@ int fleet_check(lfdm_fleet* f) {
     return LFDM_OK;
 }
 
-// Occupancies the model's integration kernels are built for (24-DOF: one wave per SIMD only).
+// Most waves per SIMD the model's one-lane integration kernels are built for.
 int max_waves(int dof) { return dof == 24 ? kMaxWaves24 : (dof == 18 ? kMaxWaves18 : kMaxWaves11); }
 
 void fleet_drop_graph(lfdm_fleet* f) {
