@@ -23,9 +23,12 @@ constexpr size_t kPart = size_t(2) << 20;
 // Below this the threads' start-up costs more than they save.
 constexpr size_t kLeast = size_t(4) << 20;
 
-std::mutex g_lock;  // guards everything here; a copy holds it, a second one at the time goes the plain way
+std::mutex g_lock;  // guards the buffers; a copy holds it, a second one at the time goes the plain way
 char* g_pinned = nullptr;  // kThreads x kBuffers parts
 char* g_small = nullptr;   // kStagedBytes
+// The holders have a lock of their own: a copy may wait for seconds of work ahead of it, and handles come
+// and go meanwhile.
+std::mutex g_holders_lock;
 int g_holders = 0;
 
 // One thread's share: every kThreads-th part.
@@ -117,13 +120,14 @@ hipError_t copy_out(void* dst, const void* device_src, size_t n, hipStream_t str
 }
 
 void copy_out_hold() {
-    std::lock_guard<std::mutex> lock(g_lock);
+    std::lock_guard<std::mutex> lock(g_holders_lock);
     ++g_holders;
 }
 
 void copy_out_release() {
-    std::lock_guard<std::mutex> lock(g_lock);
+    std::lock_guard<std::mutex> holders(g_holders_lock);
     if (--g_holders > 0) return;
+    std::lock_guard<std::mutex> lock(g_lock);  // free: a copy is made for a handle
     for (char** p : {&g_pinned, &g_small}) {
         if (*p) (void)hipHostFree(*p);
         *p = nullptr;

@@ -1,6 +1,7 @@
 """Records read back from the GPU (lfdm_get_states) through each of its ways: gathered into pinned memory
 (up to 1 MiB), copied plainly, and by several threads through pinned parts of 2 MiB (from 4 MiB on)."""
 import threading
+import time
 
 import numpy as np
 import pytest
@@ -73,3 +74,23 @@ def test_several_fleets_read_back_at_once():
     assert not wrong
     for s, _ in fleets:
         s.close()
+
+
+def test_handles_come_and_go_while_another_reads_back():
+    """A read back waits for the work ahead of it (some 1 s here); a handle made meanwhile does not."""
+    flat = lfdm_amd.params_from_json(18, W.HMMWV_VEH, W.HMMWV_TIRE)
+    s = SolverHalfImplicitGPU(18, 64)
+    s.construct_flat(flat, 64, np.array([[0.0, 0.0, 0.2, 0.0], [1.0, 0.0, 0.2, 0.0]]), TMeasy)
+    s.Initialize(s.zero_record(), 64)
+    s.set_controls_table()
+    s.advance(10)
+    s.get_states()
+    s.advance(400_000)
+    reader = threading.Thread(target=s.get_states)
+    reader.start()
+    time.sleep(0.05)
+    SolverHalfImplicitGPU(11, 1).close()
+    still_reading = reader.is_alive()
+    reader.join()
+    s.close()
+    assert still_reading
