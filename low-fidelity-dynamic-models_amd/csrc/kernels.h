@@ -35,16 +35,17 @@ constexpr int kMaxWaves11 = 4, kMaxWaves18 = 3, kMaxWaves24 = 2;
 // beyond (at 131,072 18-DOF vehicles two lanes would take two rounds of 6.1 against 10.8).  The kernels are
 // built for the wavefronts per SIMD they make, which keeps the dispatcher from stacking two on one SIMD
 // while another is idle.  One-lane fleets of w wavefronts per SIMD, w below the model's most, run the
-// kernel built for w for the same reason.
+// kernel built for w for the same reason.  one_lane: launches that have no lane-group kernels (the strict step,
+// a caller's own controls functor).
 struct KernelChoice {
     int lanes, waves;
 };
 
-inline KernelChoice choose_kernel(int dof, long long S, int simds, bool strict) {
+inline KernelChoice choose_kernel(int dof, long long S, int simds, bool one_lane) {
     const long long wf = S / kWave;
     if (simds <= 0 || wf <= 0) return {1, 0};
     const auto per = [&](int lanes) { return (wf * lanes + simds - 1) / simds; };
-    if (!strict) {
+    if (!one_lane) {
         if (dof != 11 && per(4) <= 2) return {4, (int)per(4)};
         if (per(2) <= 2) return {2, dof == 11 ? (int)per(2) : 2};
     }

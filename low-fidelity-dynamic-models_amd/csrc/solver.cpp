@@ -484,7 +484,7 @@ Launch make_launch(lfdm_solver* h, int mode, double t0, int nsteps, double cs = 
         L.step_base = (int)std::llround(t0 / h->step);
     }
     L.strict = h->arith == LFDM_ARITH_STRICT ? 1 : 0;
-    const KernelChoice c = choose_kernel(h->dof, h->S, simd_count(h), L.strict != 0);
+    const KernelChoice c = choose_kernel(h->dof, h->S, simd_count(h), L.strict != 0 || mode == kCtrlFunctor);
     L.lanes = c.lanes;
     L.waves = c.waves;
     return L;

@@ -1,5 +1,6 @@
 """Small fleets on the GPU run the lane-group kernels (two or four lanes per vehicle); results have the bits
 of the one-lane kernels, which a fleet bucket set to two waves per SIMD runs at any size."""
+import ctypes
 import os
 
 import numpy as np
@@ -9,6 +10,7 @@ from conftest import DATA
 
 import lfdm_amd
 from lfdm_amd import workloads as W
+from lfdm_amd._lib import lib
 from lfdm_amd.solver import Fleet, SolverHalfImplicitGPU, TMeasy, TMeasyNr
 
 pytestmark = pytest.mark.gpu
@@ -152,3 +154,21 @@ def test_step_jacobian_does_not_depend_on_the_fleet():
     assert torch.isfinite(ref).all()
     for n in (1, 64, 65):
         assert torch.equal(jacobian(n), ref[..., :n]), n
+
+
+@pytest.mark.parametrize("dof,n", [(11, 40_000), (18, 20_000), (18, 65_536), (24, 40_000)])
+def test_functor_launches_take_the_one_lane_occupancy(dof, n):
+    """A caller's controls functor has one-lane kernels only: one wavefront per SIMD on fleets that fill no more,
+    whatever the lane-group kernels of such a fleet are built for."""
+    s = fleet(dof, False, n)
+    size, block, grid, stream = 8, ctypes.c_int(), ctypes.c_int(), ctypes.c_void_p()
+    begin = lib.lfdm_functor_chunk_begin
+    begin.argtypes = [ctypes.c_void_p, ctypes.c_double, ctypes.c_int, ctypes.c_void_p, ctypes.c_int] + [ctypes.c_void_p] * 3
+    out = [ctypes.addressof(v) for v in (block, grid, stream)]
+    raw = (ctypes.c_char * 4096)()
+    while begin(s._h, 0.0, 1, raw, size, *out) != 0:
+        size += 8
+        assert size < 4096
+    _, waves, lanes, strict = np.frombuffer(raw, np.int32, 4, size - 16)  # the launch record's last fields
+    s.close()
+    assert (waves, lanes, strict) == (1, 1, 0)
