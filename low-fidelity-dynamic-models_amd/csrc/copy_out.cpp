@@ -94,11 +94,14 @@ char* copy_out_begin(const void* dst, size_t n) {
 void copy_out_end() { g_lock.unlock(); }
 
 hipError_t copy_out(void* dst, const void* device_src, size_t n, hipStream_t stream) {
-    std::unique_lock<std::mutex> lock(g_lock, std::defer_lock);
     int device = 0;
-    if (n < kLeast || !ordinary(dst) || hipGetDevice(&device) != hipSuccess || !lock.try_lock() ||
-        !ensure(g_pinned, kThreads * kBuffers * kPart))
-        return plain(dst, device_src, n, stream);
+    if (n < kLeast || !ordinary(dst) || hipGetDevice(&device) != hipSuccess) return plain(dst, device_src, n, stream);
+    // The source is complete before a helper is started: hipStreamPerThread names another stream in every
+    // thread, on which a helper's copy would not wait for the work ahead on the caller's.  And the buffers
+    // are not held, nor do eight threads wait, while that work runs.
+    if (const hipError_t e = hipStreamSynchronize(stream); e != hipSuccess) return e;
+    std::unique_lock<std::mutex> lock(g_lock, std::try_to_lock);
+    if (!lock || !ensure(g_pinned, kThreads * kBuffers * kPart)) return plain(dst, device_src, n, stream);
     hipError_t result[kThreads];
     std::vector<std::thread> helpers;
     int started = 1;  // this thread takes the first share

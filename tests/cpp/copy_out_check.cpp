@@ -1,0 +1,175 @@
+// Record copies to the host (csrc/copy_out.cpp) on a stand-in for the HIP runtime: streams are queues of work
+// that runs when a thread waits for it, hipStreamPerThread names another queue in every thread, and device
+// memory is host memory.  Built without the HIP library by the Makefile's `copycheck`; run by
+// tests/test_copy_out_host.py, one check per argument.
+#include "../../low-fidelity-dynamic-models_amd/csrc/copy_out.cpp"
+
+#include <chrono>
+#include <cstdio>
+#include <cstdlib>
+#include <deque>
+#include <functional>
+#include <map>
+#include <string>
+
+namespace {
+
+struct Queue {
+    std::mutex lock, running;
+    std::deque<std::function<void()>> work;
+    void add(std::function<void()> f) {
+        std::lock_guard<std::mutex> g(lock);
+        work.push_back(std::move(f));
+    }
+    // Runs the queue in order until done() (null: until it is empty).
+    void drain(const std::function<bool()>& done) {
+        std::lock_guard<std::mutex> one(running);
+        while (!done || !done()) {
+            std::function<void()> f;
+            {
+                std::lock_guard<std::mutex> g(lock);
+                if (work.empty()) return;
+                f = std::move(work.front());
+                work.pop_front();
+            }
+            f();
+        }
+    }
+};
+
+Queue& queue_of(hipStream_t s) {
+    if (s == hipStreamPerThread) {
+        static thread_local Queue own;
+        return own;
+    }
+    return *reinterpret_cast<Queue*>(s);
+}
+
+struct Event {
+    std::atomic<bool> done{true};
+    Queue* queue = nullptr;
+};
+
+std::mutex g_count_lock;
+std::map<void*, size_t> g_allocated;  // pinned blocks alive
+int g_pins = 0;                       // pinned blocks ever
+std::atomic<int> g_copies{0};         // copies asked of the runtime
+
+}  // namespace
+
+extern "C" {
+hipError_t hipSetDevice(int) { return hipSuccess; }
+hipError_t hipGetDevice(int* d) { return *d = 0, hipSuccess; }
+hipError_t hipGetLastError() { return hipSuccess; }
+hipError_t hipEventCreateWithFlags(hipEvent_t* e, unsigned) {
+    *e = reinterpret_cast<hipEvent_t>(new Event);
+    return hipSuccess;
+}
+hipError_t hipEventDestroy(hipEvent_t e) {
+    delete reinterpret_cast<Event*>(e);
+    return hipSuccess;
+}
+hipError_t hipEventRecord(hipEvent_t e, hipStream_t s) {
+    Event* ev = reinterpret_cast<Event*>(e);
+    ev->queue = &queue_of(s);
+    ev->done = false;
+    ev->queue->add([ev] { ev->done = true; });
+    return hipSuccess;
+}
+hipError_t hipEventSynchronize(hipEvent_t e) {
+    Event* ev = reinterpret_cast<Event*>(e);
+    if (ev->queue) ev->queue->drain([ev] { return ev->done.load(); });
+    return hipSuccess;
+}
+hipError_t hipStreamSynchronize(hipStream_t s) {
+    queue_of(s).drain(nullptr);
+    return hipSuccess;
+}
+hipError_t hipMemcpyAsync(void* dst, const void* src, size_t n, hipMemcpyKind, hipStream_t s) {
+    ++g_copies;
+    queue_of(s).add([=] { std::memcpy(dst, src, n); });
+    return hipSuccess;
+}
+hipError_t hipHostMalloc(void** p, size_t n, unsigned) {
+    *p = std::malloc(n);
+    std::lock_guard<std::mutex> g(g_count_lock);
+    g_allocated[*p] = n;
+    ++g_pins;
+    return hipSuccess;
+}
+hipError_t hipHostFree(void* p) {
+    std::lock_guard<std::mutex> g(g_count_lock);
+    if (!g_allocated.erase(p)) std::abort();
+    std::free(p);
+    return hipSuccess;
+}
+hipError_t hipPointerGetAttributes(hipPointerAttribute_t* a, const void*) {
+    *a = {};
+    a->type = hipMemoryTypeUnregistered;
+    return hipSuccess;
+}
+}
+
+namespace {
+
+using lfdm::copy_out;
+
+constexpr size_t kMiB = size_t(1) << 20;
+
+std::vector<char> bytes(size_t n, int seed) {
+    std::vector<char> v(n);
+    unsigned x = seed * 2654435761u + 1;
+    for (char& c : v) c = (char)((x = x * 1664525u + 1013904223u) >> 24);
+    return v;
+}
+
+// Work ahead of the copy, on the calling thread's hipStreamPerThread: every byte must come from after it.
+bool per_thread_stream() {
+    const std::vector<char> fresh = bytes(33 * kMiB + 7, 1);
+    std::vector<char> device(fresh.size(), 'x'), out(fresh.size());
+    queue_of(hipStreamPerThread).add([&] {
+        std::this_thread::sleep_for(std::chrono::milliseconds(200));
+        device = fresh;
+    });
+    return copy_out(out.data(), device.data(), out.size(), hipStreamPerThread) == hipSuccess && out == fresh;
+}
+
+// A copy that still waits for work ahead of it keeps neither the pinned parts nor the helper threads: one of a
+// finished stream meanwhile goes in parts.
+bool waiting_copy_keeps_nothing() {
+    const std::vector<char> fresh = bytes(40 * kMiB, 2);
+    std::vector<char> a(fresh.size()), b(fresh.size());
+    Queue busy, idle;
+    std::atomic<bool> reached{false}, go{false};
+    busy.add([&] {
+        reached = true;
+        while (!go) std::this_thread::yield();
+    });
+    bool ok = true;
+    std::thread waits([&] {
+        ok = copy_out(a.data(), fresh.data(), a.size(), reinterpret_cast<hipStream_t>(&busy)) == hipSuccess;
+    });
+    while (!reached) std::this_thread::yield();
+    std::this_thread::sleep_for(std::chrono::milliseconds(100));
+    const int before = g_copies;
+    const bool second = copy_out(b.data(), fresh.data(), b.size(), reinterpret_cast<hipStream_t>(&idle)) == hipSuccess;
+    const int parts = g_copies - before;
+    go = true;
+    waits.join();
+    return ok && second && a == fresh && b == fresh && parts == 20;
+}
+
+}  // namespace
+
+int main(int argc, char** argv) {
+    const std::map<std::string, bool (*)()> checks = {{"per_thread_stream", per_thread_stream},
+                                                      {"waiting_copy_keeps_nothing", waiting_copy_keeps_nothing}};
+    const auto it = checks.find(argc > 1 ? argv[1] : "");
+    if (it == checks.end()) return 2;
+    lfdm::copy_out_hold();
+    bool ok = it->second();
+    lfdm::copy_out_release();
+    ok = ok && g_allocated.empty();
+    std::printf("%s %s\n", it->first.c_str(), ok ? "ok" : "FAILED");
+    return ok ? 0 : 1;
+}
