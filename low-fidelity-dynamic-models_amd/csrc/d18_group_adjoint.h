@@ -550,8 +550,18 @@ LFDM_HD void load_carry_g(const double* p, size_t S, int q, S18gb<G>& l, K18b& k
     l.udot = b.udot; l.vdot = b.vdot; l.crank = b.crank;
 }
 
-// adj_reverse_lane on a group; c, kb: the vehicle's storage for its constants and their adjoints (its lanes
-// read and write the same values).
+// Storage of T lanes' constants and the adjoints of them.  Every lane adds every contribution to its own copy
+// of the adjoints: in one copy per vehicle an addition would count once only while the group's lanes load and
+// store it in step.  The constants, which each lane writes before it reads them, all the same values, need one.
+template <int G, int T>
+struct ReverseStore {
+    K18 c[T / G];
+    K18b kb[T];
+    LFDM_HD K18& constants(int lane) { return c[lane / G]; }
+    LFDM_HD K18b& adjoints(int lane) { return kb[lane]; }
+};
+
+// adj_reverse_lane on a group; c, kb: this lane's of a ReverseStore.
 template <int G>
 LFDM_HD void adj_reverse_group(const AdjLaunch& L, int slot, int q, const PSet& P, const MapXY* tab, K18& c, K18b& kb) {
     const size_t S = (size_t)L.S, N = (size_t)L.n_user;

@@ -34,17 +34,16 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(W, W))
     adj_forward_group<G, W == 1>(L, slot, q, *P, tab);
 }
 
-// The constants and their adjoints lie in LDS once per vehicle: in registers they would take 88 of a lane's
-// (468 instead of 370 on four lanes).
+// The constants and their adjoints lie in LDS (ReverseStore): in registers they would take 88 of a lane's
+// (468 instead of 368 on four lanes).
 template <int G>
 __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(1, 1))) void adj_reverse_g(AdjLaunch L) {
     __shared__ MapXY tab[kGroupMapEntries];
-    __shared__ K18 ks[kThreads / G];
-    __shared__ K18b kbs[kThreads / G];
+    __shared__ ReverseStore<G, kThreads> store;
     int slot, q;
     const PSet* P;
     if (!group_lane<G>(L, tab, slot, q, P)) return;
-    adj_reverse_group<G>(L, slot, q, *P, tab, ks[threadIdx.x / G], kbs[threadIdx.x / G]);
+    adj_reverse_group<G>(L, slot, q, *P, tab, store.constants(threadIdx.x), store.adjoints(threadIdx.x));
 }
 
 template <int G>

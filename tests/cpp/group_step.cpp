@@ -173,6 +173,22 @@ void adjoint_group(const PSet& P, AdjLaunch L, int nseg, int group) {
     }
 }
 
+// The reverse sweep over the whole tape with the kernel's own storage, shared as the kernel's lanes share it:
+// the lanes here are not in step.
+template <int G>
+void adjoint_group_stored(const PSet& P, AdjLaunch L, int nseg) {
+    for (int v = 0; v < L.n_user; ++v)
+        on_lanes<G>(P, [&](int q, const MapXY* tab) { adj_forward_group<G, G == 4>(L, v, q, P, tab); });
+    L.seg_hi = nseg;
+    L.seg_lo = 0;
+    for (int v = 0; v < L.n_user; ++v) {
+        ReverseStore<G, G> store;
+        on_lanes<G>(P, [&](int q, const MapXY* tab) {
+            adj_reverse_group<G>(L, v, q, P, tab, store.constants(q), store.adjoints(q));
+        });
+    }
+}
+
 void adjoint_lanes(const PSet& P, AdjLaunch L, int nseg, int group) {
     for (int v = 0; v < L.n_user; ++v) adj_forward_lane(L, v, P);
     for (int hi = nseg; hi > 0; hi -= group) {
@@ -192,7 +208,7 @@ void adjoint_lanes(const PSet& P, AdjLaunch L, int nseg, int group) {
 
 // Adjoint forward and backward of n <= 64 18-DOF vehicles on `lanes` lanes each, checkpoints every K steps and
 // `group` segments per backward group: xy[nsteps][2][n], ctrl_bar[nsteps][3][n], state_bar[75][n],
-// param_bar[7][n].
+// param_bar[7][n].  lanes -2 and -4: two and four, with the kernel's storage (group: all segments).
 extern "C" int group_adjoint_run(int lanes, const double* flat, int len, const double* ovr, const double* init, int n,
                                  int nsteps, int K, int group, const double* ctrl, const double* xy_bar, double* xy,
                                  double* ctrl_bar, double* state_bar, double* param_bar) {
@@ -230,6 +246,8 @@ extern "C" int group_adjoint_run(int lanes, const double* flat, int len, const d
     L.fwd_tape_lo = nseg - group;
     if (lanes == 4) adjoint_group<4>(P, L, nseg, group);
     else if (lanes == 2) adjoint_group<2>(P, L, nseg, group);
+    else if (lanes == -4) adjoint_group_stored<4>(P, L, nseg);
+    else if (lanes == -2) adjoint_group_stored<2>(P, L, nseg);
     else adjoint_lanes(P, L, nseg, group);
     return 0;
 }
