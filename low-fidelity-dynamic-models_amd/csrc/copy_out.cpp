@@ -25,9 +25,7 @@ constexpr size_t kLeast = size_t(4) << 20;
 
 std::mutex g_lock;  // guards the buffers; a copy holds it, a second one at the time goes the plain way
 char* g_pinned = nullptr;  // kThreads x kBuffers parts
-char* g_small = nullptr;   // kStagedBytes
-// The holders have a lock of their own: a copy may wait for seconds of work ahead of it, and handles come
-// and go meanwhile.
+// The holders have a lock of their own: handles come and go while a copy is under way.
 std::mutex g_holders_lock;
 int g_holders = 0;
 
@@ -82,16 +80,22 @@ hipError_t plain(void* dst, const void* src, size_t n, hipStream_t stream) {
 
 }  // namespace
 
-char* copy_out_begin(const void* dst, size_t n) {
-    if (n > kStagedBytes || !ordinary(dst) || !g_lock.try_lock()) return nullptr;
-    if (!ensure(g_small, kStagedBytes)) {
-        g_lock.unlock();
-        return nullptr;
-    }
-    return g_small;
+Staging::~Staging() {
+    if (p_) (void)hipHostFree(p_);
 }
 
-void copy_out_end() { g_lock.unlock(); }
+char* Staging::buffer(const void* dst, size_t n) {
+    if (n > kStagedBytes || !ordinary(dst) || !lock_.try_lock()) return nullptr;
+    if (n > n_) {
+        if (p_) (void)hipHostFree(p_);
+        p_ = nullptr;
+        n_ = ensure(p_, n) ? n : 0;
+    }
+    if (!p_) lock_.unlock();
+    return p_;
+}
+
+void Staging::done() { lock_.unlock(); }
 
 hipError_t copy_out(void* dst, const void* device_src, size_t n, hipStream_t stream) {
     int device = 0;
@@ -131,10 +135,8 @@ void copy_out_release() {
     std::lock_guard<std::mutex> holders(g_holders_lock);
     if (--g_holders > 0) return;
     std::lock_guard<std::mutex> lock(g_lock);  // free: a copy is made for a handle
-    for (char** p : {&g_pinned, &g_small}) {
-        if (*p) (void)hipHostFree(*p);
-        *p = nullptr;
-    }
+    if (g_pinned) (void)hipHostFree(g_pinned);
+    g_pinned = nullptr;
 }
 
 }  // namespace lfdm

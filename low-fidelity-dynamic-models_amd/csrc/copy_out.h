@@ -3,6 +3,7 @@
 #include <hip/hip_runtime.h>
 
 #include <cstddef>
+#include <mutex>
 
 namespace lfdm {
 
@@ -10,14 +11,27 @@ namespace lfdm {
 // there.  dst may be any memory hipMemcpy takes; ordinary host memory is the case this is for.
 hipError_t copy_out(void* dst, const void* device_src, size_t n, hipStream_t stream);
 
-// Small arrays for dst: a pinned buffer of n bytes that a kernel may write itself, the caller's until
-// copy_out_end; null where there is none (n above kStagedBytes, dst not ordinary host memory, a copy under
-// way in another thread).
+// A handle's own pinned memory for its small arrays, which a kernel may write itself.  Not shared: a read back
+// that waits for work ahead of it keeps no other handle's from its own.
 constexpr size_t kStagedBytes = size_t(1) << 20;
-char* copy_out_begin(const void* dst, size_t n);
-void copy_out_end();
+class Staging {
+public:
+    Staging() = default;
+    Staging(const Staging&) = delete;
+    Staging& operator=(const Staging&) = delete;
+    ~Staging();
+    // A buffer of n bytes for dst, the caller's until done(); null where there is none (n above kStagedBytes, dst
+    // not ordinary host memory, another thread's read back of the handle under way).
+    char* buffer(const void* dst, size_t n);
+    void done();
 
-// Solver handles hold the buffers: the last one to go frees them.
+private:
+    std::mutex lock_;
+    char* p_ = nullptr;
+    size_t n_ = 0;
+};
+
+// Solver handles hold copy_out's buffers: the last one to go frees them.
 void copy_out_hold();
 void copy_out_release();
 

@@ -151,6 +151,7 @@ struct lfdm_solver {
     int* d_which = nullptr;
     double* d_rec = nullptr;
     size_t rec_cap = 0;
+    Staging staged;  // small records on their way to the host
     std::vector<int> outs_host;  // output steps of the launch in flight (source of an async copy)
     // differentiation form
     double* d_ckpt = nullptr;
@@ -1014,12 +1015,12 @@ int lfdm_get_states(lfdm_solver* h, double* records) {
     }
     const size_t need = (size_t)h->total * h->rec;
     // a small fleet's records: gathered straight into pinned memory, without a copy of its own behind the gather
-    if (char* staged = copy_out_begin(records, need * sizeof(double))) {
+    if (char* staged = h->staged.buffer(records, need * sizeof(double))) {
         hipError_t e = launch_gather(h->d_state, h->S, h->rec, h->d_user_slot, (int)h->total,
                                      reinterpret_cast<double*>(staged), h->stream);
         if (e == hipSuccess) e = hipStreamSynchronize(h->stream);
         if (e == hipSuccess) std::memcpy(records, staged, need * sizeof(double));
-        copy_out_end();
+        h->staged.done();
         if (e != hipSuccess) return fail(LFDM_E_HIP, hipGetErrorString(e));
         return LFDM_OK;
     }

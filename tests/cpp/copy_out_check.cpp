@@ -159,11 +159,36 @@ bool waiting_copy_keeps_nothing() {
     return ok && second && a == fresh && b == fresh && parts == 20;
 }
 
+// Two handles' small read backs under way at once each have pinned memory of their own; a second one of the same
+// handle has none meanwhile.  A later, larger one has enough.
+bool small_reads_apart() {
+    std::vector<char> dst(1000);
+    lfdm::Staging a, b;
+    char* const p = a.buffer(dst.data(), dst.size());
+    char *q = nullptr, *again = p;
+    std::thread([&] {
+        q = b.buffer(dst.data(), dst.size());
+        again = a.buffer(dst.data(), dst.size());
+        if (q) std::memset(q, 2, 1000);
+        b.done();
+    }).join();
+    if (!p || !q || again) return false;
+    std::memset(p, 1, 1000);
+    a.done();
+    if (a.buffer(dst.data(), 10) != p || b.buffer(dst.data(), lfdm::kStagedBytes + 1)) return false;
+    a.done();
+    char* const large = b.buffer(dst.data(), lfdm::kStagedBytes);
+    std::memset(large, 3, lfdm::kStagedBytes);
+    b.done();
+    return true;
+}
+
 }  // namespace
 
 int main(int argc, char** argv) {
     const std::map<std::string, bool (*)()> checks = {{"per_thread_stream", per_thread_stream},
-                                                      {"waiting_copy_keeps_nothing", waiting_copy_keeps_nothing}};
+                                                      {"waiting_copy_keeps_nothing", waiting_copy_keeps_nothing},
+                                                      {"small_reads_apart", small_reads_apart}};
     const auto it = checks.find(argc > 1 ? argv[1] : "");
     if (it == checks.end()) return 2;
     lfdm::copy_out_hold();
