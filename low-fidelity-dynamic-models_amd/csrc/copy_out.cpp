@@ -22,9 +22,17 @@ constexpr int kThreads = 8, kBuffers = 2;
 constexpr size_t kPart = size_t(2) << 20;
 // Below this the threads' start-up costs more than they save.
 constexpr size_t kLeast = size_t(4) << 20;
+// Pinning the buffers costs 1 to 2 ms, more than a read of less than 30 MB saves, and a handle that is read once and
+// closed would pay it each time: they are pinned for a handle once it has read this much.  Made, run 10 steps, read
+// once and closed, pinned at once -> so: 7,000 vehicles 4.1 -> 2.5 ms, 10,000 6.0 -> 4.3, 100,003 43.9 -> 44.0.
+constexpr size_t kReadBefore = kThreads * kBuffers * kPart;
+// Likewise a handle's own small buffer, 26 us to pin and free, where a read saves 8: the first read of 64 vehicles
+// 42 -> 25 us, the fifth 16.
+constexpr int kPlainReads = 3;
 
 std::mutex g_lock;  // guards the buffers; a copy holds it, a second one at the time goes the plain way
-char* g_pinned = nullptr;  // kThreads x kBuffers parts
+char* g_pinned = nullptr;
+size_t g_parts = 0;  // parts it holds, kThreads x kBuffers at most
 // The holders have a lock of their own: handles come and go while a copy is under way.
 std::mutex g_holders_lock;
 int g_holders = 0;
@@ -34,11 +42,11 @@ hipError_t copy_parts(int device, char* dst, const char* src, size_t n, int firs
     hipError_t e = hipSetDevice(device);
     hipEvent_t done[kBuffers] = {};
     for (int b = 0; b < kBuffers && e == hipSuccess; ++b) e = hipEventCreateWithFlags(&done[b], hipEventDisableTiming);
-    char* const pinned = g_pinned + (size_t)first * kBuffers * kPart;
     const size_t parts = (n + kPart - 1) / kPart;
+    const auto pinned = [](size_t p) { return g_pinned + p % (kThreads * kBuffers) * kPart; };
     const auto size = [&](size_t p) { return std::min(kPart, n - p * kPart); };
     const auto request = [&](size_t p, int b) {
-        hipError_t r = hipMemcpyAsync(pinned + b * kPart, src + p * kPart, size(p), hipMemcpyDeviceToHost, stream);
+        hipError_t r = hipMemcpyAsync(pinned(p), src + p * kPart, size(p), hipMemcpyDeviceToHost, stream);
         return r == hipSuccess ? hipEventRecord(done[b], stream) : r;
     };
     int b = 0;
@@ -47,7 +55,7 @@ hipError_t copy_parts(int device, char* dst, const char* src, size_t n, int firs
         if (p + kThreads < parts) e = request(p + kThreads, (b + 1) % kBuffers);
         const hipError_t w = hipEventSynchronize(done[b]);
         if (e == hipSuccess) e = w;
-        if (e == hipSuccess) std::memcpy(dst + p * kPart, pinned + b * kPart, size(p));
+        if (e == hipSuccess) std::memcpy(dst + p * kPart, pinned(p), size(p));
     }
     // no request may still be writing the buffers when they go back
     if (e != hipSuccess) (void)hipStreamSynchronize(stream);
@@ -56,8 +64,10 @@ hipError_t copy_parts(int device, char* dst, const char* src, size_t n, int firs
     return e;
 }
 
-bool ensure(char*& p, size_t n) {
-    if (!p && hipHostMalloc((void**)&p, n, hipHostMallocPortable) != hipSuccess) {
+// p as n bytes of pinned memory in place of what it was.
+bool pin(char*& p, size_t n) {
+    if (p) (void)hipHostFree(p);
+    if (hipHostMalloc((void**)&p, n, hipHostMallocPortable) != hipSuccess) {
         p = nullptr;
         (void)hipGetLastError();  // the plain way is taken instead
     }
@@ -86,26 +96,28 @@ Staging::~Staging() {
 
 char* Staging::buffer(const void* dst, size_t n) {
     if (n > kStagedBytes || !ordinary(dst) || !lock_.try_lock()) return nullptr;
-    if (n > n_) {
-        if (p_) (void)hipHostFree(p_);
-        p_ = nullptr;
-        n_ = ensure(p_, n) ? n : 0;
-    }
+    if (reads_ < kPlainReads) ++reads_;
+    else if (n > n_) n_ = pin(p_, n) ? n : 0;
     if (!p_) lock_.unlock();
     return p_;
 }
 
 void Staging::done() { lock_.unlock(); }
 
-hipError_t copy_out(void* dst, const void* device_src, size_t n, hipStream_t stream) {
+hipError_t copy_out(void* dst, const void* device_src, size_t n, hipStream_t stream, size_t& before) {
     int device = 0;
-    if (n < kLeast || !ordinary(dst) || hipGetDevice(&device) != hipSuccess) return plain(dst, device_src, n, stream);
+    before = std::min(before + n, kReadBefore);
+    if (n < kLeast || before < kReadBefore || !ordinary(dst) || hipGetDevice(&device) != hipSuccess)
+        return plain(dst, device_src, n, stream);
     // The source is complete before a helper is started: hipStreamPerThread names another stream in every
     // thread, on which a helper's copy would not wait for the work ahead on the caller's.  And the buffers
     // are not held, nor do eight threads wait, while that work runs.
     if (const hipError_t e = hipStreamSynchronize(stream); e != hipSuccess) return e;
     std::unique_lock<std::mutex> lock(g_lock, std::try_to_lock);
-    if (!lock || !ensure(g_pinned, kThreads * kBuffers * kPart)) return plain(dst, device_src, n, stream);
+    if (!lock) return plain(dst, device_src, n, stream);
+    const size_t parts = std::min<size_t>((n + kPart - 1) / kPart, kThreads * kBuffers);
+    if (parts > g_parts) g_parts = pin(g_pinned, parts * kPart) ? parts : 0;
+    if (!g_pinned) return plain(dst, device_src, n, stream);
     hipError_t result[kThreads];
     std::vector<std::thread> helpers;
     int started = 1;  // this thread takes the first share
@@ -137,6 +149,7 @@ void copy_out_release() {
     std::lock_guard<std::mutex> lock(g_lock);  // free: a copy is made for a handle
     if (g_pinned) (void)hipHostFree(g_pinned);
     g_pinned = nullptr;
+    g_parts = 0;
 }
 
 }  // namespace lfdm

@@ -8,8 +8,9 @@
 namespace lfdm {
 
 // Copies n bytes from device memory to dst after the work pending on `stream`, and returns when they are
-// there.  dst may be any memory hipMemcpy takes; ordinary host memory is the case this is for.
-hipError_t copy_out(void* dst, const void* device_src, size_t n, hipStream_t stream);
+// there.  dst may be any memory hipMemcpy takes; ordinary host memory is the case this is for.  before: what
+// the handle has read so far (0 at its start), counted here.
+hipError_t copy_out(void* dst, const void* device_src, size_t n, hipStream_t stream, size_t& before);
 
 // A handle's own pinned memory for its small arrays, which a kernel may write itself.  Not shared: a read back
 // that waits for work ahead of it keeps no other handle's from its own.
@@ -21,7 +22,7 @@ public:
     Staging& operator=(const Staging&) = delete;
     ~Staging();
     // A buffer of n bytes for dst, the caller's until done(); null where there is none (n above kStagedBytes, dst
-    // not ordinary host memory, another thread's read back of the handle under way).
+    // not ordinary host memory, another thread's read back of the handle under way, the handle's first reads).
     char* buffer(const void* dst, size_t n);
     void done();
 
@@ -29,6 +30,7 @@ private:
     std::mutex lock_;
     char* p_ = nullptr;
     size_t n_ = 0;
+    int reads_ = 0;
 };
 
 // Solver handles hold copy_out's buffers: the last one to go frees them.

@@ -152,6 +152,7 @@ struct lfdm_solver {
     double* d_rec = nullptr;
     size_t rec_cap = 0;
     Staging staged;  // small records on their way to the host
+    size_t bytes_read = 0;  // copy_out's count
     std::vector<int> outs_host;  // output steps of the launch in flight (source of an async copy)
     // differentiation form
     double* d_ckpt = nullptr;
@@ -1027,7 +1028,7 @@ int lfdm_get_states(lfdm_solver* h, double* records) {
     if (int rc = ensure_buffer(h->d_rec, h->rec_cap, need)) return rc;
     hipError_t e = launch_gather(h->d_state, h->S, h->rec, h->d_user_slot, (int)h->total, h->d_rec, h->stream);
     if (e != hipSuccess) return fail(LFDM_E_HIP, hipGetErrorString(e));
-    HIPCHK(copy_out(records, h->d_rec, need * sizeof(double), h->stream));
+    HIPCHK(copy_out(records, h->d_rec, need * sizeof(double), h->stream, h->bytes_read));
     return LFDM_OK;
 }
 

@@ -112,9 +112,14 @@ hipError_t hipPointerGetAttributes(hipPointerAttribute_t* a, const void*) {
 
 namespace {
 
-using lfdm::copy_out;
 
 constexpr size_t kMiB = size_t(1) << 20;
+
+// A copy for a handle that has read nothing before.
+hipError_t copy_out(void* dst, const void* src, size_t n, hipStream_t stream) {
+    size_t before = 0;
+    return lfdm::copy_out(dst, src, n, stream, before);
+}
 
 std::vector<char> bytes(size_t n, int seed) {
     std::vector<char> v(n);
@@ -164,6 +169,9 @@ bool waiting_copy_keeps_nothing() {
 bool small_reads_apart() {
     std::vector<char> dst(1000);
     lfdm::Staging a, b;
+    for (int i = 0; i < 4; ++i)
+        for (lfdm::Staging* s : {&a, &b})
+            if (s->buffer(dst.data(), dst.size())) s->done();
     char* const p = a.buffer(dst.data(), dst.size());
     char *q = nullptr, *again = p;
     std::thread([&] {
@@ -183,12 +191,49 @@ bool small_reads_apart() {
     return true;
 }
 
+// A handle that reads little before it goes pins nothing.
+bool read_once_pins_nothing() {
+    std::vector<char> small(1000), large(5 * kMiB), device(5 * kMiB, 'd');
+    Queue idle;
+    lfdm::Staging handle;
+    size_t before = 0;
+    for (int i = 0; i < 2; ++i) {
+        if (handle.buffer(small.data(), small.size())) handle.done();
+        if (lfdm::copy_out(large.data(), device.data(), large.size(), reinterpret_cast<hipStream_t>(&idle), before) !=
+                hipSuccess ||
+            large != device)
+            return false;
+    }
+    return g_pins == 0;
+}
+
+// One that goes on reading pins what its reads need, once; a larger read of another handle then pins more.
+bool later_reads_pin_once() {
+    Queue idle;
+    size_t first = 0, second = 0;
+    const auto read = [&](size_t n, size_t& before) {
+        const std::vector<char> device = bytes(n, (int)n);
+        std::vector<char> out(n);
+        return lfdm::copy_out(out.data(), device.data(), n, reinterpret_cast<hipStream_t>(&idle), before) == hipSuccess &&
+               out == device;
+    };
+    bool ok = true;
+    for (int i = 0; i < 12; ++i) ok = ok && read(5 * kMiB + 1, first);
+    ok = ok && g_pins == 1 && g_allocated.begin()->second == 6 * kMiB;
+    ok = ok && read(19 * kMiB, second) && g_pins == 1;  // this handle's first: the plain way
+    ok = ok && read(19 * kMiB, second) && g_pins == 2 && g_allocated.begin()->second == 20 * kMiB;
+    ok = ok && read(70 * kMiB + 3, second) && g_pins == 3 && g_allocated.begin()->second == 32 * kMiB;
+    return ok && read(5 * kMiB, first) && g_pins == 3 && g_allocated.size() == 1;
+}
+
 }  // namespace
 
 int main(int argc, char** argv) {
     const std::map<std::string, bool (*)()> checks = {{"per_thread_stream", per_thread_stream},
                                                       {"waiting_copy_keeps_nothing", waiting_copy_keeps_nothing},
-                                                      {"small_reads_apart", small_reads_apart}};
+                                                      {"small_reads_apart", small_reads_apart},
+                                                      {"read_once_pins_nothing", read_once_pins_nothing},
+                                                      {"later_reads_pin_once", later_reads_pin_once}};
     const auto it = checks.find(argc > 1 ? argv[1] : "");
     if (it == checks.end()) return 2;
     lfdm::copy_out_hold();
