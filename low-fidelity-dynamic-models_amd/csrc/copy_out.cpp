@@ -5,6 +5,8 @@
 // overlap.
 #include "copy_out.h"
 
+#include <sched.h>
+
 #include <algorithm>
 #include <atomic>
 #include <cstring>
@@ -26,8 +28,11 @@ constexpr size_t kLeast = size_t(4) << 20;
 // closed would pay it each time: they are pinned for a handle once it has read this much.  Made, run 10 steps, read
 // once and closed, pinned at once -> so: 7,000 vehicles 4.1 -> 2.5 ms, 10,000 6.0 -> 4.3, 100,003 43.9 -> 44.0.
 constexpr size_t kReadBefore = kThreads * kBuffers * kPart;
-// Likewise a handle's own small buffer, 26 us to pin and free, where a read saves 8: the first read of 64 vehicles
-// 42 -> 25 us, the fifth 16.
+// A process on one CPU, whose threads only take turns, copies no less than this in parts either: 100,003 vehicles 6.2 ->
+// 5.4 ms there, but 30,000 1.35 -> 1.43 and 10,000 0.45 -> 0.53 (on two CPUs 6.2 -> 3.2, 1.31 -> 0.95, 0.45 -> 0.37).
+constexpr size_t kLeastOneCpu = kReadBefore;
+// A handle's own small buffer takes 26 us to pin and free, where a read saves 8: the first read of 64 vehicles 42 ->
+// 25 us, the fifth 16.
 constexpr int kPlainReads = 3;
 
 std::mutex g_lock;  // guards the buffers; a copy holds it, a second one at the time goes the plain way
@@ -83,6 +88,11 @@ bool ordinary(const void* dst) {
     return true;
 }
 
+bool one_cpu() {
+    cpu_set_t mine;
+    return sched_getaffinity(0, sizeof(mine), &mine) == 0 && CPU_COUNT(&mine) == 1;
+}
+
 hipError_t plain(void* dst, const void* src, size_t n, hipStream_t stream) {
     const hipError_t e = hipMemcpyAsync(dst, src, n, hipMemcpyDeviceToHost, stream);
     return e == hipSuccess ? hipStreamSynchronize(stream) : e;
@@ -107,7 +117,8 @@ void Staging::done() { lock_.unlock(); }
 hipError_t copy_out(void* dst, const void* device_src, size_t n, hipStream_t stream, size_t& before) {
     int device = 0;
     before = std::min(before + n, kReadBefore);
-    if (n < kLeast || before < kReadBefore || !ordinary(dst) || hipGetDevice(&device) != hipSuccess)
+    if (n < (one_cpu() ? kLeastOneCpu : kLeast) || before < kReadBefore || !ordinary(dst) ||
+        hipGetDevice(&device) != hipSuccess)
         return plain(dst, device_src, n, stream);
     // The source is complete before a helper is started: hipStreamPerThread names another stream in every
     // thread, on which a helper's copy would not wait for the work ahead on the caller's.  And the buffers

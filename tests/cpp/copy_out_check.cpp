@@ -4,6 +4,8 @@
 // tests/test_copy_out_host.py, one check per argument.
 #include "../../low-fidelity-dynamic-models_amd/csrc/copy_out.cpp"
 
+#include <sched.h>
+
 #include <chrono>
 #include <cstdio>
 #include <cstdlib>
@@ -226,6 +228,27 @@ bool later_reads_pin_once() {
     return ok && read(5 * kMiB, first) && g_pins == 3 && g_allocated.size() == 1;
 }
 
+// A process on one CPU, where helper threads only take turns, copies 18 MB the plain way and 60 MB in parts.
+bool one_cpu() {
+    cpu_set_t all, one;
+    sched_getaffinity(0, sizeof(all), &all);
+    CPU_ZERO(&one);
+    for (int c = 0; c < CPU_SETSIZE && CPU_COUNT(&one) == 0; ++c)
+        if (CPU_ISSET(c, &all)) CPU_SET(c, &one);
+    sched_setaffinity(0, sizeof(one), &one);
+    Queue idle;
+    bool ok = true;
+    for (size_t n : {size_t(18000000), size_t(60000000)}) {
+        const std::vector<char> device = bytes(n, 9);
+        std::vector<char> out(n);
+        const int copies = g_copies;
+        size_t before = 100 * kMiB;
+        ok = ok && lfdm::copy_out(out.data(), device.data(), n, reinterpret_cast<hipStream_t>(&idle), before) == hipSuccess &&
+             out == device && g_copies - copies == (n == 18000000 ? 1 : 29);
+    }
+    return ok;
+}
+
 }  // namespace
 
 int main(int argc, char** argv) {
@@ -233,7 +256,8 @@ int main(int argc, char** argv) {
                                                       {"waiting_copy_keeps_nothing", waiting_copy_keeps_nothing},
                                                       {"small_reads_apart", small_reads_apart},
                                                       {"read_once_pins_nothing", read_once_pins_nothing},
-                                                      {"later_reads_pin_once", later_reads_pin_once}};
+                                                      {"later_reads_pin_once", later_reads_pin_once},
+                                                      {"one_cpu", one_cpu}};
     const auto it = checks.find(argc > 1 ? argv[1] : "");
     if (it == checks.end()) return 2;
     lfdm::copy_out_hold();
