@@ -66,7 +66,7 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(1, 1))
 
 // One wavefront per (row, 64 slots), the rows with most work first, each row through the parts of the step it
 // reaches.  With a vehicle's 21 rows on one lane the kernel took the latency of 21 sweeps at any size and ran a
-// fleet of 1,563 wavefronts in two rounds: 64 vehicles 580 -> 27 us, 100,003 vehicles 2,479 -> 410 us (0.98 TB/s
+// fleet of 1,563 wavefronts in two rounds: 64 vehicles 580 -> 27 us, 100,003 vehicles 2,479 -> 428 us (0.94 TB/s
 // of Jacobian).  One wave per SIMD (330 VGPRs): two, with 102 spilled, measure the same.
 __global__ __launch_bounds__(kWave) __attribute__((amdgpu_waves_per_eu(1, 1))) void step_jacobian(AdjLaunch L) {
     const int slot = blockIdx.x * kWave + threadIdx.x;

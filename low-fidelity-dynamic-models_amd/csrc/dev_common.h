@@ -38,6 +38,15 @@ LFDM_HD void opaque(double& v) {
 
 __device__ __forceinline__ int uniform(int v) { return __builtin_amdgcn_readfirstlane(v); }
 
+// Whether b holds on any of the wavefront's active lanes, the same answer on all of them (host: this lane's).
+LFDM_HD bool any_lane(bool b) {
+#if defined(__HIP_DEVICE_COMPILE__)
+    return __builtin_amdgcn_ballot_w64(b) != 0;
+#else
+    return b;
+#endif
+}
+
 // Quotient and square root of the step code.  On the device: Newton-Raphson refinement of the
 // hardware reciprocal v_rcp_f64 (two iterations, then the quotient with one remainder correction,
 // Markstein's method) and of the reciprocal square root v_rsq_f64 (Goldschmidt-style coupled
