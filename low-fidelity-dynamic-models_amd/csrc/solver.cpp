@@ -1593,12 +1593,16 @@ int fleet_end(lfdm_fleet* f) {
 // at once, each fills the chip by itself, and running the buckets side by side only mixes kernels of
 // different register and LDS budgets on the CUs (the 2,000,000-vehicle mixed 11/18/24-DOF fleet: 1.47
 // s side by side, 1.42 s one after another).  Smaller buckets run side by side, filling the chip
-// together.
+// together, and so do buckets on lane groups, which make two wavefronts per SIMD at most and leave VALU cycles
+// that another bucket's can use, even where each makes as many as its kernels allow (1,000 steps side by side and
+// chained: two of 65,536 18-DOF vehicles 11.6 and 12.1 ms, 65,536 of 18 and 24 DOF 13.0 and 13.6, two of 16,384
+// 5.2 and 5.3).
 bool fleet_serial(lfdm_fleet* f, const std::vector<std::vector<Launch>>& ls) {
     if (f->buckets.size() < 2) return false;
     for (size_t b = 0; b < f->buckets.size(); ++b) {
         lfdm_solver* h = f->buckets[b];
         const long long simds = simd_count(h);
+        if (!ls[b].empty() && ls[b][0].lanes > 1) return false;
         const int w = (!ls[b].empty() && ls[b][0].waves > 0) ? ls[b][0].waves : max_waves(h->dof);
         if (simds <= 0 || (long long)(h->S / kWave) < simds * w) return false;
     }
