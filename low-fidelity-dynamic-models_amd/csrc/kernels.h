@@ -31,6 +31,8 @@ constexpr int kMaxWaves11 = 4, kMaxWaves18 = 3, kMaxWaves24 = 2;
 //   18-DOF  16,384 vehicles  7.8 / 4.0 / 2.5    32,768  8.1 / 4.2 / 4.1    65,536  8.3 / 6.1 / 7.7
 //   24-DOF  16,384 vehicles  9.9 / 5.4 / 3.2    32,768 10.3 / 5.3 / 4.9    65,536 10.3 / 8.3 / 9.8
 //   11-DOF  16,384 vehicles  4.9 / 2.4          32,768  5.5 / 2.4          65,536  5.7 / 3.9
+// TMeasyNr fleets, whose tires take longer, gain likewise (65,536 vehicles, one / two: 18-DOF 11.7 / 9.5, 24-DOF 13.0 /
+// 11.0, 11-DOF 7.3 / 5.4; 16,384, one / four: 18-DOF 11.6 / 3.4, 24-DOF 12.6 / 3.9).
 // So: four lanes while they make at most two wavefronts per SIMD, two lanes while they do, and one lane
 // beyond (at 131,072 18-DOF vehicles two lanes would take two rounds of 6.1 against 10.8).  The kernels are
 // built for the wavefronts per SIMD they make, which keeps the dispatcher from stacking two on one SIMD
