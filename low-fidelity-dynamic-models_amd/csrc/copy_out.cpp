@@ -145,7 +145,10 @@ hipError_t copy_out(void* dst, const void* device_src, size_t n, hipStream_t str
         result[k] = copy_parts(device, (char*)dst, (const char*)device_src, n, k, stream);
     for (std::thread& t : helpers) t.join();
     for (hipError_t e : result)
-        if (e != hipSuccess) return e;
+        if (e != hipSuccess) {  // what failed (an event, say) the plain way may not need
+            (void)hipGetLastError();
+            return plain(dst, device_src, n, stream);
+        }
     return hipSuccess;
 }
 

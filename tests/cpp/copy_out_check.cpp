@@ -56,6 +56,7 @@ std::mutex g_count_lock;
 std::map<void*, size_t> g_allocated;  // pinned blocks alive
 int g_pins = 0;                       // pinned blocks ever
 std::atomic<int> g_copies{0};         // copies asked of the runtime
+std::atomic<int> g_events_left{1 << 30};  // events the runtime can still make
 
 }  // namespace
 
@@ -64,6 +65,7 @@ hipError_t hipSetDevice(int) { return hipSuccess; }
 hipError_t hipGetDevice(int* d) { return *d = 0, hipSuccess; }
 hipError_t hipGetLastError() { return hipSuccess; }
 hipError_t hipEventCreateWithFlags(hipEvent_t* e, unsigned) {
+    if (g_events_left-- <= 0) return hipErrorOutOfMemory;
     *e = reinterpret_cast<hipEvent_t>(new Event);
     return hipSuccess;
 }
@@ -249,6 +251,20 @@ bool one_cpu() {
     return ok;
 }
 
+// Without events for some of the parts the copy is made the plain way, which needs none.
+bool no_events() {
+    Queue idle;
+    const std::vector<char> device = bytes(40 * kMiB, 4);
+    for (int left : {0, 5, 15}) {
+        g_events_left = left;
+        std::vector<char> out(device.size());
+        if (copy_out(out.data(), device.data(), out.size(), reinterpret_cast<hipStream_t>(&idle)) != hipSuccess ||
+            out != device)
+            return false;
+    }
+    return true;
+}
+
 }  // namespace
 
 int main(int argc, char** argv) {
@@ -257,7 +273,8 @@ int main(int argc, char** argv) {
                                                       {"small_reads_apart", small_reads_apart},
                                                       {"read_once_pins_nothing", read_once_pins_nothing},
                                                       {"later_reads_pin_once", later_reads_pin_once},
-                                                      {"one_cpu", one_cpu}};
+                                                      {"one_cpu", one_cpu},
+                                                      {"no_events", no_events}};
     const auto it = checks.find(argc > 1 ? argv[1] : "");
     if (it == checks.end()) return 2;
     lfdm::copy_out_hold();

@@ -10,7 +10,7 @@ CHECK = os.path.join(ROOT, "low-fidelity-dynamic-models_amd", "lfdm_amd", "copy_
 
 
 @pytest.mark.parametrize("name", ["per_thread_stream", "waiting_copy_keeps_nothing", "small_reads_apart",
-                                  "read_once_pins_nothing", "later_reads_pin_once", "one_cpu"])
+                                  "read_once_pins_nothing", "later_reads_pin_once", "one_cpu", "no_events"])
 def test_copy_out(name):
     assert os.path.exists(CHECK), "run make -C low-fidelity-dynamic-models_amd copycheck"
     r = subprocess.run([CHECK, name], capture_output=True, text=True, timeout=60)
